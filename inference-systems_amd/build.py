@@ -56,6 +56,7 @@ SOURCES = [
     "gemm_fp32.hip",
     "gemm_direct.hip",
     "gemm_staged.hip",
+    "gemm_wide.hip",
     "gemm_decode.hip",
     "gemm_gemv.hip",
     "gemm_argmax.hip",

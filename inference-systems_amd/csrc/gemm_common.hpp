@@ -452,6 +452,9 @@ int launch_fp32_naive(const Problem& p, hipStream_t s);
 int launch_fp32_tiled(const Problem& p, hipStream_t s);
 int launch_mfma_direct(const Problem& p, hipStream_t s);
 int launch_mfma_staged(const Problem& p, hipStream_t s);
+// mfma_staged's 256 x 256 tiles (gemm_wide.hip) and the grids that take them.
+bool mfma_wide_pays(const Problem& p);
+int launch_mfma_wide(const Problem& p, hipStream_t s);
 int launch_splitk_decode(const Problem& p, hipStream_t s);
 int launch_gemv_decode(const Problem& p, hipStream_t s);
 
