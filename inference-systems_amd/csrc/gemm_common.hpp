@@ -451,6 +451,9 @@ __device__ __forceinline__ void grouped_tile(int t, int tiles_m, int tiles_n, in
 int launch_fp32_naive(const Problem& p, hipStream_t s);
 int launch_fp32_tiled(const Problem& p, hipStream_t s);
 int launch_mfma_direct(const Problem& p, hipStream_t s);
+// mfma_direct's form for rows that are no aligned 16-byte chunks (gemm_ragged.hip).
+bool mfma_ragged_ok(const Problem& p);
+int launch_mfma_ragged(const Problem& p, hipStream_t s);
 int launch_mfma_staged(const Problem& p, hipStream_t s);
 // mfma_staged's 256 x 256 tiles (gemm_wide.hip) and the grids that take them.
 bool mfma_wide_pays(const Problem& p);

@@ -5,7 +5,10 @@
 // gemm_wmma.cu:56-104 with B = W[N,K]) and also covers what they skip:
 // partial tiles (gemm_bench.cu:92), K that is not a multiple of 16, odd
 // strides and unaligned pointers.  It is the selection table's fallback for
-// any half-precision problem the faster kernels cannot take.
+// any half-precision problem the faster kernels cannot take: those run
+// gemm_ragged.hip's tiles, and only rows shorter than one 16-byte chunk (K or,
+// on B[K,N], N below 8) the kernel here, which also runs any problem asked of
+// it by name.
 #include "gemm_common.hpp"
 
 namespace nvg {
@@ -143,9 +146,17 @@ int launch_typed(const Problem& p, hipStream_t s) {
     return check_launch("mfma_direct");
 }
 
+// Every row of A and B starts and ends on a 16-byte chunk: the problems
+// mfma_staged takes, which come here only by name.
+bool chunked_rows(const Problem& p) {
+    return reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.b) % 16 == 0 && p.lda % 8 == 0 &&
+           p.ldb % 8 == 0 && p.k % 8 == 0 && (p.b_layout == NANOVLLM_GEMM_B_NK || p.n % 8 == 0);
+}
+
 }  // namespace
 
 int launch_mfma_direct(const Problem& p, hipStream_t s) {
+    if (!chunked_rows(p) && mfma_ragged_ok(p)) return launch_mfma_ragged(p, s);
     if (p.dtype_in == NANOVLLM_GEMM_BF16) {
         if (p.dtype_out == NANOVLLM_GEMM_BF16) return launch_typed<NANOVLLM_GEMM_BF16, NANOVLLM_GEMM_BF16>(p, s);
         return launch_typed<NANOVLLM_GEMM_BF16, NANOVLLM_GEMM_F32>(p, s);
