@@ -58,6 +58,7 @@ SOURCES = [
     "gemm_staged.hip",
     "gemm_wide.hip",
     "gemm_ragged.hip",
+    "gemm_narrow.hip",
     "gemm_decode.hip",
     "gemm_gemv.hip",
     "gemm_argmax.hip",

@@ -455,6 +455,9 @@ int launch_mfma_direct(const Problem& p, hipStream_t s);
 bool mfma_ragged_ok(const Problem& p);
 int launch_mfma_ragged(const Problem& p, hipStream_t s);
 int launch_mfma_staged(const Problem& p, hipStream_t s);
+// mfma_staged's 32-row tiles (gemm_narrow.hip) and the grids that take them.
+bool mfma_narrow_pays(const Problem& p);
+int launch_mfma_narrow(const Problem& p, hipStream_t s);
 // mfma_staged's 256 x 256 tiles (gemm_wide.hip) and the grids that take them.
 bool mfma_wide_pays(const Problem& p);
 int launch_mfma_wide(const Problem& p, hipStream_t s);

@@ -8,8 +8,8 @@
 //     grid, 64 x 64 each), K-tiles of 64 elements; grids with enough
 //     128 x 256 tiles for every CU take those (8 waves in a 2x4 grid, 64 x
 //     64 each), grids of at most 128 tiles of 128 x 128 (half the CUs) take
-//     64 x 64 tiles (waves of 32 x 32), and large grids the 256 x 256 tiles
-//     of gemm_wide.hip;
+//     64 x 64 tiles (waves of 32 x 32), smaller ones the tiles of
+//     gemm_narrow.hip, and large grids the 256 x 256 tiles of gemm_wide.hip;
 //   * operands move global -> LDS with global_load_lds_dwordx4 (no VGPR
 //     staging) into a ring of STAGES tile buffers; tiles t+1 .. t+STAGES-1
 //     are in flight while tile t is multiplied, and each wave waits on its
@@ -555,14 +555,13 @@ int launch_tile(const Problem& p, hipStream_t s) {
 // Tile and schedule by grid size (bf16, MI355X, one launch; every choice
 // sums K in the same order, so none changes a result bit).  "tiles" counts
 // 128 x 128 tiles, "wide" 128 x 256 ones:
-//   * tiles <= 128 (half the CUs): 64 x 64 tiles, four times the workgroups
-//     (1024^3 11.7 -> 6.8 us, 512 x 4096 x 1024 12.3 -> 8.1 us,
-//     2048 x 1024 x 2048 20.6 -> 13.8 us, 512 x 1024 x 3584 33.0 -> 17.0 us),
-//     on a 3-deep ring with spread copies (against a 2-deep burst ring:
-//     1024^3 6.85 -> 6.57 us, 512 x 4096 x 1024 8.49 -> 8.04, 256 x 6144 x
-//     1024 8.03 -> 7.46, 2048 x 1024 x 2048 14.2 -> 14.0, 512 x 1024 x 3584
-//     27.3 -> 17.2); SiLU pairs take 64 x 128, also with spread copies on
-//     a 3-deep ring;
+//   * grids of at most one round of 64 x 64 tiles (SiLU pairs: two of 64 x
+//     32 outputs): the smaller tiles of gemm_narrow.hip, by the rules there;
+//   * tiles <= 128 (half the CUs) above that: 64 x 64 tiles, four times the
+//     workgroups (512 x 4096 x 1024 12.3 -> 8.1 us, 2048 x 1024 x 2048 20.6 ->
+//     13.8 us), on a 3-deep ring with spread copies (against a 2-deep burst
+//     ring: 512 x 4096 x 1024 8.49 -> 8.04, 256 x 6144 x 1024 8.03 -> 7.46,
+//     2048 x 1024 x 2048 14.2 -> 14.0);
 //   * 128 < wide <= 256 or wide > 384: one 8-wave workgroup per CU on
 //     128 x 256 (half the A reads of two 128 x 128 tiles), 3-deep ring,
 //     copies spread between the MFMAs.  Against the 2-deep 128 x 128 burst
@@ -587,18 +586,8 @@ int launch_epi(const Problem& p, hipStream_t s) {
     // A fused gate/up tile covers half its W rows in output columns.
     const int64_t n_tiles = EPI == EPI_SILU_MUL ? 2 * p.n : p.n;
     const int64_t tiles = ((p.m + 127) / 128) * ((n_tiles + 127) / 128);
-    if (tiles <= kSmallGridTiles) {
-        if constexpr (EPI == EPI_NONE) {
-            return launch_tile<DT, DT_OUT, 64, 64, 2, 2, 3, EPI, RS, 1>(p, s);
-        } else if constexpr (EPI == EPI_SILU_MUL) {
-            // gate/up pairs need two 32-row W blocks per wave: 64 x 128
-            // tiles, spread copies on a 3-deep ring (gate_up n = 3584, K =
-            // 1024, M = 96 / 128 / 256: 9.4 / 9.4-9.7 / 9.6-10.5 -> 8.7 /
-            // 8.6-8.9 / 8.8-9.4 us against the 2-deep burst ring, and
-            // 15.7-17.0 -> 14.5-14.8 us at K = 2048 against the 3-deep one)
-            return launch_tile<DT, DT_OUT, 64, 128, 2, 2, 3, EPI, RS, 1>(p, s);
-        }
-    }
+    if constexpr (EPI == EPI_NONE)
+        if (tiles <= kSmallGridTiles) return launch_tile<DT, DT_OUT, 64, 64, 2, 2, 3, EPI, RS, 1>(p, s);
     if constexpr (EPI != EPI_ARGMAX) {
         const int64_t wide = ((p.m + 127) / 128) * ((n_tiles + 255) / 256);
         if (wide > kCus / 2 && (wide <= kCus || wide > 3 * kCus / 2))
@@ -642,6 +631,7 @@ int launch_typed(const Problem& p, hipStream_t s) {
 
 int launch_mfma_staged(const Problem& p, hipStream_t s) {
     if (mfma_wide_pays(p)) return launch_mfma_wide(p, s);
+    if (mfma_narrow_pays(p)) return launch_mfma_narrow(p, s);
     if (p.epi == EPI_ARGMAX) {
         constexpr int F = NANOVLLM_GEMM_F32;
         if (p.dtype_in == NANOVLLM_GEMM_BF16) return launch_epi<NANOVLLM_GEMM_BF16, F, EPI_ARGMAX>(p, s);
