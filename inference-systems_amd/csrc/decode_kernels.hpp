@@ -67,7 +67,7 @@ constexpr bool decode_cfg_fits() {
 // W fragments (8 consecutive k of one column per lane) are read back with
 // gfx950's transposing LDS read, two ds_read_b64_tr_b16 of 4 k-rows each.
 template <int DT, int DT_OUT, int AROWS, int RG, int WAVES, int LPB, int PARTS, int EPI, int PRO, int KN = 0,
-          int AREG = 0>
+          int AREG = 0, int RB = 0>
 __global__ __launch_bounds__(WAVES * 64) void splitk_decode_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, void* __restrict__ c,
     int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, uint64_t* __restrict__ keys,
@@ -104,17 +104,36 @@ __global__ __launch_bounds__(WAVES * 64) void splitk_decode_kernel(
     const int r8 = lane >> 3;    // copy: row within the instruction's 8
     const int chunk = (lane & 7) ^ r8;   // copy: chunk of the line this lane fetches
 
+    // Workgroup `nblk` of those along N.  RB: rows of A beyond AROWS go to
+    // further workgroups along y; the grid is 8 x row blocks x N blocks / 8,
+    // which puts the workgroups that read the same W rows on one XCD
+    // (workgroup w runs on XCD w % 8), next to each other.  A form of its own:
+    // the extra indexes at the start cost every small launch 0.1-0.2 us.
+    static_assert(!RB || EPI != EPI_ARGMAX, "the LM heads run in one row of workgroups");
+    int nblk = blockIdx.x;
+    if constexpr (RB) {
+        nblk += kNumXcd * blockIdx.z;
+        const int64_t row0 = int64_t(blockIdx.y) * AROWS;
+        a += row0 * lda;
+        c = static_cast<char*>(c) + row0 * ldc * (DT_OUT == NANOVLLM_GEMM_F32 ? 4 : 2);
+        m = min_i64(m - row0, AROWS);
+        if constexpr (PRO != PRO_NONE) pro.a2 += row0 * pro.lda2;
+        if constexpr (PRO == PRO_ADD_NORM) pro.res_out += row0 * pro.ldres;
+    }
+
     // EPI_SILU_MUL: W-row groups pair up, group 2s holding gate rows and
     // group 2s + 1 the up rows of the same 16 output columns.
     static_assert(EPI != EPI_SILU_MUL || RG % 2 == 0, "gate/up group pairs");
     constexpr int OG = EPI == EPI_SILU_MUL ? RG / 2 : RG;   // 16-column output groups per workgroup
+    const uint32_t nblks = RB ? uint32_t((n + 16 * OG - 1) / (16 * OG)) : gridDim.x;
+    if (RB && uint32_t(nblk) >= nblks) return;   // the last of 8 along x
     // Consecutive column blocks go to consecutive workgroups, which the
     // hardware hands to the 8 XCDs round robin.  Giving each XCD a contiguous
     // run of blocks instead (xcd_remap, so the two workgroups writing one
     // 128-byte output line share an L2) measured 0.3 us slower on every
     // decode shape (N = 6144, K = 1024, M = 1-64; 1024 x 3584): W streams
     // better when each XCD's reads spread over the whole matrix.
-    const int64_t n0 = int64_t(blockIdx.x) * 16 * OG;         // first output column
+    const int64_t n0 = int64_t(nblk) * 16 * OG;               // first output column
     const uint16_t* wsrc[IW];
 #pragma unroll
     for (int h = 0; h < IW; ++h) {
@@ -361,10 +380,10 @@ __global__ __launch_bounds__(WAVES * 64) void splitk_decode_kernel(
                         const int64_t kc = line * kLine + (4 * st + grp) * 8;
                         const bool in_k = kc < k;
                         const u32x4_t wv = in_k ? nwv[t][st] : u32x4_t{0u, 0u, 0u, 0u};
-                        // Every workgroup forms s for all of A; line L's new residual is
-                        // written by workgroup L mod gridDim.x.
+                        // Every workgroup forms s for its rows of A; line L's new
+                        // residual is written by workgroup L mod nblks.
                         const bool writes =
-                            __builtin_amdgcn_readfirstlane(int(uint32_t(line) % gridDim.x)) == int(blockIdx.x);
+                            __builtin_amdgcn_readfirstlane(int(uint32_t(line) % nblks)) == nblk;
 #pragma unroll
                         for (int g = 0; g < MG; ++g) {
                             u32x4_t res;
@@ -518,17 +537,22 @@ __global__ __launch_bounds__(WAVES * 64) void splitk_decode_kernel(
 }
 
 template <int DT, int DT_OUT, int AROWS, int RG, int WAVES, int LPB, int PARTS, int EPI, int PRO = PRO_NONE,
-          int KN = 0, int AREG = 0>
+          int KN = 0, int AREG = 0, int RB = 0>
 int launch_cfg(const Problem& p, hipStream_t s) {
     constexpr int OG = EPI == EPI_SILU_MUL ? RG / 2 : RG;
-    if (p.m > AROWS) return set_error(NANOVLLM_GEMM_EUNSUPPORTED, "splitk_decode: M above the configuration's rows");
-    const int64_t blocks = (p.n + 16 * OG - 1) / (16 * OG);
-    if (blocks > INT32_MAX) return set_error(NANOVLLM_GEMM_EINVAL, "splitk_decode: grid too large");
-    const dim3 grid(static_cast<uint32_t>(blocks)), block(WAVES * 64);
+    if (!RB && p.m > AROWS)
+        return set_error(NANOVLLM_GEMM_EUNSUPPORTED, "splitk_decode: M above the configuration's rows");
+    const int64_t blocks = (p.n + 16 * OG - 1) / (16 * OG), row_blocks = (p.m + AROWS - 1) / AROWS;
+    if (blocks > INT32_MAX || row_blocks > 65535 || (RB && blocks > 8 * 65535)) return set_error(NANOVLLM_GEMM_EINVAL, "splitk_decode: grid too large");
+    const dim3 block(WAVES * 64);
+    dim3 grid(static_cast<uint32_t>(blocks));
+    if (RB)
+        grid = dim3(kNumXcd, static_cast<uint32_t>(row_blocks), static_cast<uint32_t>((blocks + kNumXcd - 1) / kNumXcd));
     if (EPI == EPI_ARGMAX) *p.key_blocks = blocks;
     const ProArgs pro{static_cast<const uint16_t*>(p.a2), p.lda2, p.group, p.group_stride,
                       static_cast<const uint16_t*>(p.norm_w), p.eps, static_cast<uint16_t*>(p.res_out), p.ldres};
-    hipLaunchKernelGGL((splitk_decode_kernel<DT, DT_OUT, AROWS, RG, WAVES, LPB, PARTS, EPI, PRO, KN, AREG>), grid, block, 0, s,
+    hipLaunchKernelGGL((splitk_decode_kernel<DT, DT_OUT, AROWS, RG, WAVES, LPB, PARTS, EPI, PRO, KN, AREG, RB>),
+                       grid, block, 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.c, p.m, p.n, p.k,
                        p.lda, p.ldb, p.ldc, p.keys, pro, p.sample);
     return check_launch("splitk_decode");

@@ -43,23 +43,25 @@ namespace {
 //     and these copies alone 4.01 us (M = 8) / 4.58 us (M = 32); an empty
 //     kernel costs 1.56 us per graph node.  With at most 2048 rows (N = 1024, K = 3584,
 //     the down and output projections) 16 rows per workgroup give twice the
-//     workgroups, with 16 waves along K up to M = 16 (M = 1 / 16 / 32: 4.7 /
-//     6.6 / 8.5 us, against 7.0 / 9.0 / 11.7 us with 32 rows).
+//     workgroups, with 16 waves along K (M = 1 / 16: 4.7 / 6.6 us, against
+//     7.0 / 9.0 us with 32 rows).  Where that leaves CUs idle, the rows of A
+//     are spread over workgroups too (launch_rows);
 //   * rows >= 65536 (the LM head, N = 151936, K = 1024): M = 1 runs the
 //     register-loading kernel (48.4 us; with a prologue, the M <= 8
 //     configuration); M = 8 / 16 / 32: 53.5 / 57.5 / 63.9 us (61.2 / 65.7 /
 //     75.8 us with register loading).
 //   * 33 <= M <= 64 (the plain GEMM only, below 65536 rows): A's copies now
-//     outweigh W's, so 8 waves and 8 K partitions in every configuration,
-//     16 / 32 / 48 rows per workgroup up to 4096 / 8192 / 65535 rows.
-//     Against mfma_staged, whose 64 x 64 tiles leave most CUs idle on these
-//     grids (bf16, M = 64, K = 1024 unless given): N = 1024 3.6 against
-//     5.9 us, 1024 x K 3584 6.5 / 15.5, 2048 x K 2048 4.8 / 9.7, 3584 3.8 /
-//     6.0, 4096 x K 4096 10.0 / 19.0, 6144 4.6 / 6.0, 8224 5.7 / 6.2; from
-//     16384 rows mfma_staged's larger grid wins (7.1 against 9.9 us), and
-//     the selection table sends M > 32 there.
+//     outweigh W's, so 8 waves and 8 K partitions above 2048 rows, 16 / 32 /
+//     48 rows per workgroup up to 4096 / 8192 / 65535 rows; from 16384 rows
+//     mfma_staged's larger grid wins (7.1 against 9.9 us), and the selection
+//     table sends M > 32 there.
 // A prologue adds its own copies per line to the same configurations.
 constexpr int64_t kWideN = 65536;
+
+constexpr int64_t kDecodeCus = 256;
+
+// W rows up to which a workgroup takes 16 of them (not SiLU pairs).
+constexpr int64_t kNarrowRows = 2048;
 
 // 33 <= M <= 64 below 65536 rows: the plain GEMM, and SiLU-and-mul on
 // gate/up row-group pairs (32 rows per workgroup).
@@ -70,13 +72,19 @@ int launch_rows64(const Problem& p, hipStream_t s) {
     if constexpr (EPI == EPI_SILU_MUL) {
         return launch_cfg<DT, DT_OUT, 64, 2, 8, 1, 8, EPI>(p, s);
     } else {
+        // Up to kNarrowRows, 16 or 32 rows of A per workgroup, whichever first
+        // fits the CUs (W from HBM, M = 64, us, 64 rows / this: N = 1024, K =
+        // 3584 11.4 / 6.7; 2048 x K 2048 7.8 / 6.4).
+        if (rows <= kNarrowRows) {
+            const int64_t wgs = (rows + 15) / 16;
+            if (wgs * ((p.m + 15) / 16) <= kDecodeCus) return launch_cfg<DT, DT_OUT, 16, 1, 8, 2, 8, EPI, PRO_NONE, 0, 0, 1>(p, s);
+            return launch_cfg<DT, DT_OUT, 32, 1, 8, 1, 8, EPI, PRO_NONE, 0, 0, 1>(p, s);
+        }
         if (rows <= 4096) return launch_cfg<DT, DT_OUT, 64, 1, 8, 1, 8, EPI>(p, s);
         if (rows <= 8192) return launch_cfg<DT, DT_OUT, 64, 2, 8, 1, 8, EPI>(p, s);
         return launch_cfg<DT, DT_OUT, 64, 3, 8, 1, 8, EPI>(p, s);
     }
 }
-
-constexpr int64_t kDecodeCus = 256;
 
 // Workgroups of a configuration resident on one CU at once (LDS, waves and
 // registers), from the runtime's occupancy query, once per configuration.
@@ -150,6 +158,21 @@ int launch_picked(const Problem& p, hipStream_t s, int64_t rows) {
     return rc;
 }
 
+// launch_rows' choices below the wide ones, on AROWS rows of A per workgroup.
+template <int DT, int DT_OUT, int EPI, int AROWS, int PRO>
+int launch_row_blocks(const Problem& p, hipStream_t s) {
+    if constexpr (EPI != EPI_SILU_MUL)
+        if (p.n <= kNarrowRows) return launch_cfg<DT, DT_OUT, AROWS, 1, 16, 1, 16, EPI, PRO, 0, 0, 1>(p, s);
+    return launch_cfg<DT, DT_OUT, AROWS, 2, 16, 1, 16, EPI, PRO, 0, 0, 1>(p, s);
+}
+
+// Workgroups along N below the wide choices.
+template <int EPI>
+int64_t narrow_blocks(int64_t rows) {
+    const int64_t per = EPI != EPI_SILU_MUL && rows <= kNarrowRows ? 16 : 32;
+    return (rows + per - 1) / per;
+}
+
 template <int DT, int DT_OUT, int EPI, int AROWS, int PRO>
 int launch_rows(const Problem& p, hipStream_t s) {
     const int64_t rows = EPI == EPI_SILU_MUL ? 2 * p.n : p.n;
@@ -166,11 +189,40 @@ int launch_rows(const Problem& p, hipStream_t s) {
         else if constexpr (AROWS == 16) return launch_cfg<DT, DT_OUT, 16, 2, 8, 1, 8, EPI, PRO>(p, s);
         else return launch_cfg<DT, DT_OUT, 8, 2, 8, 2, 8, EPI, PRO>(p, s);
     }
+    // Fewer rows of A per workgroup while the workgroups fit the CUs at one
+    // each: every workgroup then copies (and gates or normalises) fewer rows
+    // beside its W rows, which further workgroups read again, from L2 (they sit
+    // on one XCD: with SiLU pairs n = 1600, K = 1024, M = 24 6.45 us against 6.97
+    // in plain grid order).  W streamed from HBM, bf16, us:
+    //   * plain, 16 W rows: N = 1024, K = 3584, M = 32 / 16: 8 rows of A 5.75
+    //     / 5.75, 16 rows 6.63 / 6.69, 32 rows 8.92; N = 2048, K = 2048, M =
+    //     16: 8 rows 4.74, 16 rows 5.18; M = 32: 16 rows (256 workgroups)
+    //     5.09, 8 rows (512) 6.31, 32 rows 6.43;
+    //   * gate, N = 1024, K = 2048, M = 32: 8 rows 6.39, 16 rows 8.62, 32 rows
+    //     15.95;
+    //   * norm, N = 2000, K = 1024, M = 32: 16 rows 5.87; with SiLU pairs, n =
+    //     1024, K = 1024, M = 32 / 16: 8 rows 5.64 / 5.64, 16 rows 6.32 / 6.33,
+    //     32 rows 8.04.
+    if constexpr (EPI != EPI_ARGMAX && AROWS > 8) {
+        const int64_t wgs = narrow_blocks<EPI>(rows);
+        if (wgs * ((p.m + 7) / 8) <= kDecodeCus) return launch_row_blocks<DT, DT_OUT, EPI, 8, PRO>(p, s);
+        if constexpr (AROWS > 16)
+            if (wgs * ((p.m + 15) / 16) <= kDecodeCus) return launch_row_blocks<DT, DT_OUT, EPI, 16, PRO>(p, s);
+    }
     if constexpr (EPI != EPI_SILU_MUL) {
-        if (rows <= 2048) {
-            if constexpr (AROWS == 32) return launch_cfg<DT, DT_OUT, 32, 1, 8, 1, 16, EPI, PRO>(p, s);
-            else return launch_cfg<DT, DT_OUT, AROWS, 1, 16, 1, 16, EPI, PRO>(p, s);
+        if (rows <= kNarrowRows) {
+            // (32 rows of A are the LM head's alone here: others found 16 above.)
+            if constexpr (AROWS < 32) return launch_cfg<DT, DT_OUT, AROWS, 1, 16, 1, 16, EPI, PRO>(p, s);
+            else if constexpr (EPI == EPI_ARGMAX) return launch_cfg<DT, DT_OUT, 32, 1, 8, 1, 16, EPI, PRO>(p, s);
         }
+    }
+    // SiLU pairs behind the norm, 17 <= M <= 32: 16 rows of A on 32 pairs, as
+    // many workgroups as 32 rows on 16 and half the norm's work in each (K =
+    // 1024, M = 32: n = 2496 7.90 against 8.23 us, 3584 8.12 / 8.51; K = 1408, n =
+    // 2496 9.42 / 10.02).
+    if constexpr (EPI == EPI_SILU_MUL && PRO == PRO_ADD_NORM && AROWS == 32) {
+        if ((p.n + 31) / 32 * 2 <= kDecodeCus)
+            return launch_cfg<DT, DT_OUT, 16, 4, 8, 1, 16, EPI, PRO, 0, 0, 1>(p, s);
     }
     // Above 2048 rows (plain store, LM-head epilogues, prologues): 32 W rows
     // per 16-wave workgroup while those workgroups fit the 256 CUs at one
