@@ -227,17 +227,24 @@ __global__ __launch_bounds__(kT32Threads) void fp32_tiled_kernel(
 //   * MFMA step s of a K-tile takes k = STEPS (l / LH) + s in lane l, LH the
 //     lanes per k group of the instruction, so a lane's A (and W[N,K])
 //     values of a K-tile are one run of contiguous floats (ds_read_b128).
-// Two configurations (measured on MI355X against the 8-wave copy-into-LDS
-// kernel this replaces, in one process, fp32, B[K,N] unless noted):
-//   * 64 x 32 tiles (wave tiles of 32 x 16: two 16 x 16 blocks, so two
-//     independent v_mfma_f32_16x16x4_f32 chains per wave), BK = 64, while
-//     the grid has fewer than 512 tiles of 64 x 64: two workgroups per CU
-//     on 1024^3, so one's barrier waits hide under the other's MFMAs
-//     (1024^3 21.7 -> 19.5 us; W[N,K] 21.5 -> 19.3 us);
-//   * 64 x 64 tiles, v_mfma_f32_32x32x2_f32 in two accumulator chains (odd
+// Configurations by grid size (fp32, W[N,K] unless noted, us).  The first three
+// run v_mfma_f32_16x16x4_f32 with K split over two wave groups (BK = 64): a
+// wave then has half the MFMA chain of a K-tile, and the two partial sums come
+// closer to the exact one (relative error at K = 1024 4.1e-7 against 5.7e-7 of
+// one chain).  Fewer than 512 tiles of 64 x 64 leave CUs idle or bound by the
+// chain of MFMAs over rows past M, so tiles are as small as two workgroups to a
+// CU allow; against the 64 x 32 tiles that took all of these grids before:
+//   * 16 x 32, up to 512 of them: 16 x 6144 x 1024 12.3 -> 6.8 (32 x 32 8.1), 8
+//     x 1024 x 4096 35.6 -> 13.5, 100 x 1024 x 1024 11.6 -> 6.1, 2 x 15808 x
+//     8128 138 -> 98, 64 x 4096 x 1024 12.6 -> 8.4;
+//   * 32 x 32, up to 512: 200 x 2048 x 1024 13.0 -> 12.0 (16 x 32 12.7), 512 x
+//     1024 x 1024 12.4 -> 11.6 (32 x 64 11.9);
+//   * 32 x 64: 1024^3 19.8 -> 19.2, B[K,N] 21.7 -> 20.9, 300 x 4096 x 1024 28.9 ->
+//     28.3;
+//   * from 512 tiles of 64 x 64: 64 x 64 tiles, v_mfma_f32_32x32x2_f32 in two accumulator chains (odd
 //     steps in the second, added before the store), BK = 32, on larger grids
 //     (2048^3 156.7 -> 126.6 us, 4096^3 1208.6 -> 966.6 us).
-// Measured beside them: 64 x 64 tiles with one chain, BK = 32, 20.6 / 148.4
+// Measured beside the last: 64 x 64 tiles with one chain, BK = 32, 20.6 / 148.4
 // / 959.6 us; 32 x 32 tiles, BK = 64, 19.2-20.8 / 143 / 1107 us; one
 // K-tile of loads in flight more or less, half a K-tile of MFMAs after the
 // barrier instead of a quarter, or capping the waves per SIMD at 2-4, moved
@@ -258,12 +265,15 @@ __device__ __forceinline__ int fp32_row_swizzle(int r, int chunks) {
     return chunks == 16 ? ((r & 15) ^ (((r >> 2) & 1) << 3)) : ((r >> 1) & 7);
 }
 
-template <int BL, int BM, int BN, int BK, int MI, int CHN>
+// KW: wave groups along K.  1: the 4 waves form a 2 x 2 grid over the tile; 2:
+// a 1 x 2 grid, twice, each group taking half of every lane's run of k of a
+// K-tile, and group 1's sums are added to group 0's through LDS at the end.
+template <int BL, int BM, int BN, int BK, int MI, int CHN, int KW>
 __global__ __launch_bounds__(256) void fp32_buffered_kernel(
     const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c,
     int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n) {
     constexpr int NT = 256;
-    constexpr int WM = BM / 2, WN = BN / 2;             // wave tile
+    constexpr int WM = BM * KW / 2, WN = BN / 2;        // wave tile
     constexpr int NBA = WM / MI, NBB = WN / MI;          // MI x MI blocks of the wave tile
     static_assert(NBA >= 1 && NBB >= 1 && WM % MI == 0 && WN % MI == 0, "wave tile");
     constexpr int ACH = BK / 4;                          // 16-byte chunks per row of a K-tile (A, W[N,K])
@@ -273,14 +283,15 @@ __global__ __launch_bounds__(256) void fp32_buffered_kernel(
     constexpr int LPT = STAGE / NT;                      // loads per thread per K-tile
     constexpr int LA = A_CH / NT;                        // of which A
     static_assert(LPT * NT == STAGE && LA * NT == A_CH, "whole loads per thread");
-    constexpr int STEPS = MI == 32 ? BK / 2 : BK / 4;    // MFMA K-steps per K-tile
+    constexpr int RUN = MI == 32 ? BK / 2 : BK / 4;      // a lane's run of k in a K-tile
+    constexpr int STEPS = RUN / KW;                      // MFMA K-steps of a wave per K-tile
     constexpr int LH = MI == 32 ? 32 : 16;               // lanes per k group of the MFMA
     __shared__ u32x4_t lds[2 * STAGE];
     auto kswz = [](int kr) { return (KCH / 2) * ((kr >> 4) & 1); };
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = KW == 1 ? wave >> 1 : 0, wn = wave & 1, wk = KW == 1 ? 0 : wave >> 1;
     int tm, tn;
     grouped_tile(xcd_remap(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, 8, tm, tn);
     const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
@@ -346,7 +357,7 @@ __global__ __launch_bounds__(256) void fp32_buffered_kernel(
             const int r = wm * WM + MI * i + frow;
 #pragma unroll
             for (int q = 0; q < STEPS / 4; ++q) {
-                const int ch = (STEPS / 4) * fh + q;
+                const int ch = (RUN / 4) * fh + (STEPS / 4) * wk + q;
                 fa[i].q[q] = __builtin_bit_cast(f32x4_t, tile[r * ACH + (ch ^ fp32_row_swizzle(r, ACH))]);
             }
         }
@@ -357,13 +368,13 @@ __global__ __launch_bounds__(256) void fp32_buffered_kernel(
                 const float* bt = reinterpret_cast<const float*>(tile + A_CH);
 #pragma unroll
                 for (int s = 0; s < STEPS; ++s) {
-                    const int kr = STEPS * fh + s;
+                    const int kr = RUN * fh + STEPS * wk + s;
                     fb[i].q[s / 4][s % 4] = bt[kr * BN + (((col >> 2) ^ kswz(kr)) << 2) + (col & 3)];
                 }
             } else {
 #pragma unroll
                 for (int q = 0; q < STEPS / 4; ++q) {
-                    const int ch = (STEPS / 4) * fh + q;
+                    const int ch = (RUN / 4) * fh + (STEPS / 4) * wk + q;
                     fb[i].q[q] = __builtin_bit_cast(f32x4_t, tile[A_CH + col * ACH + (ch ^ fp32_row_swizzle(col, ACH))]);
                 }
             }
@@ -500,6 +511,24 @@ __global__ __launch_bounds__(256) void fp32_buffered_kernel(
 #pragma unroll
             for (int j = 0; j < NBA; ++j) acc[0][i][j] += acc[1][i][j];
     }
+    if constexpr (KW == 2) {
+        // Every wave has read its last fragments; the LDS tile is free.
+        static_assert(CHN == 1 && MI == 16 && 2 * NBB * NBA * 64 <= 2 * STAGE, "exchange fits in the LDS tile");
+        u32x4_t* xch = lds + wn * NBB * NBA * 64;
+        __syncthreads();
+        if (wk == 1) {
+#pragma unroll
+            for (int i = 0; i < NBB; ++i)
+#pragma unroll
+                for (int j = 0; j < NBA; ++j) xch[(i * NBA + j) * 64 + lane] = __builtin_bit_cast(u32x4_t, acc[0][i][j]);
+        }
+        __syncthreads();
+        if (wk == 1) return;
+#pragma unroll
+        for (int i = 0; i < NBB; ++i)
+#pragma unroll
+            for (int j = 0; j < NBA; ++j) acc[0][i][j] += __builtin_bit_cast(f32x4_t, xch[(i * NBA + j) * 64 + lane]);
+    }
     // acc[0][i][j][v]: MI = 32: D[n = 8 (v / 4) + 4 (l / 32) + v % 4][m = l % 32];
     // MI = 16: D[n = 4 (l / 16) + v][m = l % 16] of block (i, j): 4 adjacent
     // output columns of one row per quad.
@@ -545,10 +574,10 @@ int launch_fp32_naive(const Problem& p, hipStream_t s) {
 
 namespace {
 
-template <int BL, int BM, int BN, int BK, int MI, int CHN>
+template <int BL, int BM, int BN, int BK, int MI, int CHN, int KW = 1>
 void launch_buffered(const Problem& p, hipStream_t s) {
     const int64_t tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
-    hipLaunchKernelGGL((fp32_buffered_kernel<BL, BM, BN, BK, MI, CHN>), dim3(static_cast<uint32_t>(tiles_m * tiles_n)),
+    hipLaunchKernelGGL((fp32_buffered_kernel<BL, BM, BN, BK, MI, CHN, KW>), dim3(static_cast<uint32_t>(tiles_m * tiles_n)),
                        dim3(256), 0, s, static_cast<const float*>(p.a), static_cast<const float*>(p.b),
                        static_cast<float*>(p.c), p.m, p.n, p.k, p.lda, p.ldb, p.ldc, int(tiles_m), int(tiles_n));
 }
@@ -556,7 +585,10 @@ void launch_buffered(const Problem& p, hipStream_t s) {
 template <int BL>
 void launch_buffered_for(const Problem& p, hipStream_t s) {
     const int64_t tiles64 = ((p.m + 63) / 64) * ((p.n + 63) / 64);
-    if (tiles64 < 512) launch_buffered<BL, 64, 32, 64, 16, 1>(p, s);
+    const auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
+    if (tiles(16, 32) <= 512) launch_buffered<BL, 16, 32, 64, 16, 1, 2>(p, s);
+    else if (tiles(32, 32) <= 512) launch_buffered<BL, 32, 32, 64, 16, 1, 2>(p, s);
+    else if (tiles64 < 512) launch_buffered<BL, 32, 64, 64, 16, 1, 2>(p, s);
     else launch_buffered<BL, 64, 64, 32, 32, 2>(p, s);
 }
 
