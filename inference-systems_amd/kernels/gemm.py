@@ -101,7 +101,7 @@ def _launch(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype], 
 
 
 # ---------------------------------------------------------------------------
-# Registration of nanovllm::gemm / nanovllm::gemm_kn
+# Registration of the ops (all but sigmoid_gate, which is a custom_op)
 # ---------------------------------------------------------------------------
 # Two registrations of the same schemas over the same C ABI:
 #   torch_library  csrc/torch_ops.cpp, a TORCH_LIBRARY fragment built into
@@ -182,6 +182,15 @@ else:
     _gemm_kn_op.register_fake(_gemm_kn_fake)
 
 
+def register_op(name: str, impl, fake) -> None:
+    """nanovllm::<name>: its C++ implementation (csrc/torch_ops.cpp) or, with
+    the custom_op registration, ``impl`` over ctypes; ``fake`` either way."""
+    if REGISTRATION == "torch_library":
+        torch.library.register_fake(f"nanovllm::{name}")(fake)
+    else:
+        torch.library.custom_op(f"nanovllm::{name}", impl, mutates_args=()).register_fake(fake)
+
+
 def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """a @ w.T on the MI355X kernels (w in nn.Linear [N, K] layout)."""
     return torch.ops.nanovllm.gemm(a, w, out_dtype)
@@ -254,12 +263,10 @@ def _launch_silu_mul(a: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch
     return out
 
 
-@torch.library.custom_op("nanovllm::gemm_silu_mul", mutates_args=())
 def _gemm_silu_mul_op(a: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     return _launch_silu_mul(a, w, out_dtype)
 
 
-@_gemm_silu_mul_op.register_fake
 def _gemm_silu_mul_fake(a: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     torch._check(w.dim() == 2)
     torch._check(w.shape[0] % 2 == 0)
@@ -267,6 +274,9 @@ def _gemm_silu_mul_fake(a: torch.Tensor, w: torch.Tensor, out_dtype: Optional[to
     torch._check(a.dtype == w.dtype)
     torch._check(a.device == w.device)
     return a.new_empty((*a.shape[:-1], w.shape[0] // 2), dtype=a.dtype if out_dtype is None else out_dtype)
+
+
+register_op("gemm_silu_mul", _gemm_silu_mul_op, _gemm_silu_mul_fake)
 
 
 def gemm_silu_mul(a: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
@@ -346,13 +356,11 @@ def _launch_argmax(a: torch.Tensor, w: torch.Tensor, logits_dtype: Optional[torc
     return tokens, logits
 
 
-@torch.library.custom_op("nanovllm::gemm_argmax", mutates_args=())
 def _gemm_argmax_op(a: torch.Tensor, w: torch.Tensor,
                     logits_dtype: Optional[torch.dtype] = None) -> tuple[torch.Tensor, torch.Tensor]:
     return _launch_argmax(a, w, logits_dtype)
 
 
-@_gemm_argmax_op.register_fake
 def _gemm_argmax_fake(a: torch.Tensor, w: torch.Tensor,
                       logits_dtype: Optional[torch.dtype] = None) -> tuple[torch.Tensor, torch.Tensor]:
     torch._check(w.dim() == 2)
@@ -360,6 +368,9 @@ def _gemm_argmax_fake(a: torch.Tensor, w: torch.Tensor,
     torch._check(a.dtype == w.dtype)
     torch._check(a.device == w.device)
     return (a.new_empty(a.shape[:-1], dtype=torch.int64), a.new_empty(a.shape[:-1], dtype=torch.float32))
+
+
+register_op("gemm_argmax", _gemm_argmax_op, _gemm_argmax_fake)
 
 
 def gemm_argmax(a: torch.Tensor, w: torch.Tensor,
@@ -421,13 +432,11 @@ def _launch_sample(a: torch.Tensor, w: torch.Tensor, temperatures: torch.Tensor,
     return tokens, scores
 
 
-@torch.library.custom_op("nanovllm::gemm_sample", mutates_args=())
 def _gemm_sample_op(a: torch.Tensor, w: torch.Tensor, temperatures: torch.Tensor, seed: int,
                     offset: int, logits_dtype: Optional[torch.dtype] = None) -> tuple[torch.Tensor, torch.Tensor]:
     return _launch_sample(a, w, temperatures, seed, offset, logits_dtype)
 
 
-@_gemm_sample_op.register_fake
 def _gemm_sample_fake(a: torch.Tensor, w: torch.Tensor, temperatures: torch.Tensor, seed: int,
                       offset: int, logits_dtype: Optional[torch.dtype] = None) -> tuple[torch.Tensor, torch.Tensor]:
     torch._check(w.dim() == 2)
@@ -436,6 +445,9 @@ def _gemm_sample_fake(a: torch.Tensor, w: torch.Tensor, temperatures: torch.Tens
     torch._check(a.device == w.device)
     torch._check(temperatures.shape == a.shape[:-1])
     return (a.new_empty(a.shape[:-1], dtype=torch.int64), a.new_empty(a.shape[:-1], dtype=torch.float32))
+
+
+register_op("gemm_sample", _gemm_sample_op, _gemm_sample_fake)
 
 
 def _as_i64(x: int) -> int:
@@ -483,6 +495,22 @@ def _torch_linear(x, weight, bias, out_dtype):
     return y if out_dtype is None or y.dtype == out_dtype else y.to(out_dtype)
 
 
+def run_hip(op, reason, *args):
+    """``op(*args)`` for backend = "hip".  The op checks its contract itself,
+    so ``reason(*args)`` is asked only for the message once it has refused
+    (and for operands not on the GPU, whose fake implementation would run)."""
+    if all(t.is_cuda for t in args if isinstance(t, torch.Tensor)):
+        try:
+            return op(*args)
+        except RuntimeError:
+            why = reason(*args)
+            if why is None:
+                raise
+    else:
+        why = reason(*args)
+    raise RuntimeError(f"HIP GEMM backend is unavailable: {why}")
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *,
            out_dtype: Optional[torch.dtype] = None, backend: Optional[str] = None) -> torch.Tensor:
     """Drop-in for ``F.linear(x, weight, bias)`` with a backend switch.
@@ -494,12 +522,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     backend = validate_gemm_backend(backend) if backend is not None else default_backend()
     if backend == "torch":
         return _torch_linear(x, weight, bias, out_dtype)
-    reason = contract_reason(x, weight, out_dtype)
-    if reason is not None:
-        if backend == "auto":
-            return _torch_linear(x, weight, bias, out_dtype)
-        raise RuntimeError(f"HIP GEMM backend is unavailable: {reason}")
-    y = gemm(x, weight, out_dtype)
+    if backend == "auto" and contract_reason(x, weight, out_dtype) is not None:
+        return _torch_linear(x, weight, bias, out_dtype)
+    y = run_hip(torch.ops.nanovllm.gemm, contract_reason, x, weight, out_dtype)
     if bias is not None:
         y = y + bias.to(y.dtype)
     return y
@@ -520,12 +545,9 @@ def silu_mul_linear(x: torch.Tensor, weight: torch.Tensor, *, backend: Optional[
     backend = validate_gemm_backend(backend) if backend is not None else default_backend()
     if backend == "torch":
         return _torch_silu_mul(x, weight)
-    reason = silu_mul_contract_reason(x, weight)
-    if reason is not None:
-        if backend == "auto":
-            return _torch_silu_mul(x, weight)
-        raise RuntimeError(f"HIP GEMM backend is unavailable: {reason}")
-    return gemm_silu_mul(x, weight)
+    if backend == "auto" and silu_mul_contract_reason(x, weight) is not None:
+        return _torch_silu_mul(x, weight)
+    return run_hip(gemm_silu_mul, silu_mul_contract_reason, x, weight)
 
 
 def _torch_logits(x, weight, logits_dtype):
@@ -546,12 +568,8 @@ def greedy_linear(x: torch.Tensor, weight: torch.Tensor, *, backend: Optional[st
     logits in the model dtype, as the reference does; torch.float32 ranks
     fp32 logits."""
     backend = validate_gemm_backend(backend) if backend is not None else default_backend()
-    if backend != "torch":
-        reason = argmax_contract_reason(x, weight)
-        if reason is None:
-            return gemm_argmax(x, weight, logits_dtype)
-        if backend == "hip":
-            raise RuntimeError(f"HIP GEMM backend is unavailable: {reason}")
+    if backend == "hip" or (backend == "auto" and argmax_contract_reason(x, weight) is None):
+        return run_hip(lambda a, w: gemm_argmax(a, w, logits_dtype), argmax_contract_reason, x, weight)
     logits = _torch_logits(x, weight, logits_dtype)
     tokens = logits.argmax(dim=-1)
     return tokens, logits.gather(-1, tokens.unsqueeze(-1)).squeeze(-1)
@@ -579,10 +597,7 @@ def sample_linear(x: torch.Tensor, weight: torch.Tensor, temperatures: torch.Ten
     ``auto`` the fused head when its contract holds.  Returns (tokens,
     scores)."""
     backend = validate_gemm_backend(backend) if backend is not None else default_backend()
-    if backend != "torch":
-        reason = sample_contract_reason(x, weight, temperatures)
-        if reason is None:
-            return gemm_sample(x, weight, temperatures, seed, offset, logits_dtype)
-        if backend == "hip":
-            raise RuntimeError(f"HIP GEMM backend is unavailable: {reason}")
+    if backend == "hip" or (backend == "auto" and sample_contract_reason(x, weight, temperatures) is None):
+        return run_hip(lambda a, w, t: gemm_sample(a, w, t, seed, offset, logits_dtype), sample_contract_reason,
+                       x, weight, temperatures)
     return torch_sampler(_torch_logits(x, weight, logits_dtype), temperatures), None

@@ -34,7 +34,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _lib
-from .gemm import _CODE, default_backend, validate_gemm_backend
+from .gemm import _CODE, default_backend, register_op, run_hip, validate_gemm_backend
 
 _HALF = (torch.float16, torch.bfloat16)
 
@@ -114,17 +114,18 @@ def _launch_gated(a, gate, w, out_dtype, kernel=None):
     return out
 
 
-@torch.library.custom_op("nanovllm::gemm_gated", mutates_args=())
 def _gemm_gated_op(a: torch.Tensor, gate: torch.Tensor, w: torch.Tensor,
                    out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     return _launch_gated(a, gate, w, out_dtype)
 
 
-@_gemm_gated_op.register_fake
 def _gemm_gated_fake(a, gate, w, out_dtype=None):
     torch._check(w.dim() == 2)
     torch._check(a.dim() >= 2)
     return a.new_empty((a.shape[0], w.shape[0]), dtype=a.dtype if out_dtype is None else out_dtype)
+
+
+register_op("gemm_gated", _gemm_gated_op, _gemm_gated_fake)
 
 
 def gemm_gated(a: torch.Tensor, gate: torch.Tensor, w: torch.Tensor,
@@ -228,18 +229,19 @@ def _launch_add_rmsnorm(h, residual, norm_weight, w, eps, silu_mul, out_dtype, k
     return out, residual_out
 
 
-@torch.library.custom_op("nanovllm::gemm_add_rmsnorm", mutates_args=())
 def _gemm_add_rmsnorm_op(h: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Tensor, w: torch.Tensor,
                          eps: float, silu_mul: bool = False,
                          out_dtype: Optional[torch.dtype] = None) -> tuple[torch.Tensor, torch.Tensor]:
     return _launch_add_rmsnorm(h, residual, norm_weight, w, eps, silu_mul, out_dtype)
 
 
-@_gemm_add_rmsnorm_op.register_fake
 def _gemm_add_rmsnorm_fake(h, residual, norm_weight, w, eps, silu_mul=False, out_dtype=None):
     torch._check(h.dim() == 2 and w.dim() == 2)
     n = w.shape[0] // 2 if silu_mul else w.shape[0]
     return (h.new_empty((h.shape[0], n), dtype=h.dtype if out_dtype is None else out_dtype), torch.empty_like(h))
+
+
+register_op("gemm_add_rmsnorm", _gemm_add_rmsnorm_op, _gemm_add_rmsnorm_fake)
 
 
 def gemm_add_rmsnorm(h: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Tensor, w: torch.Tensor,
@@ -271,12 +273,8 @@ def gated_linear(x: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, *,
                  backend: Optional[str] = None) -> torch.Tensor:
     """F.linear(x * sigmoid(gate), weight) with the backend switch of ``linear``."""
     backend = validate_gemm_backend(backend) if backend is not None else default_backend()
-    if backend != "torch":
-        reason = gated_contract_reason(x, gate, weight)
-        if reason is None:
-            return gemm_gated(x, gate, weight)
-        if backend == "hip":
-            raise RuntimeError(f"HIP GEMM backend is unavailable: {reason}")
+    if backend == "hip" or (backend == "auto" and gated_contract_reason(x, gate, weight) is None):
+        return run_hip(gemm_gated, gated_contract_reason, x, gate, weight)
     return _torch_gated(x, gate, weight)
 
 
@@ -295,12 +293,11 @@ def add_rmsnorm_linear(h: torch.Tensor, residual: torch.Tensor, norm_weight: tor
     """(F.linear(norm(h + residual), weight) [then SiluAndMul], new residual)
     with the backend switch of ``linear``."""
     backend = validate_gemm_backend(backend) if backend is not None else default_backend()
-    if backend != "torch":
-        reason = add_rmsnorm_contract_reason(h, residual, norm_weight, weight, silu_mul)
-        if reason is None:
-            return gemm_add_rmsnorm(h, residual, norm_weight, weight, eps, silu_mul)
-        if backend == "hip":
-            raise RuntimeError(f"HIP GEMM backend is unavailable: {reason}")
+    if backend == "hip" or (backend == "auto" and
+                            add_rmsnorm_contract_reason(h, residual, norm_weight, weight, silu_mul) is None):
+        return run_hip(lambda a, r, nw, w: gemm_add_rmsnorm(a, r, nw, w, eps, silu_mul),
+                       lambda a, r, nw, w: add_rmsnorm_contract_reason(a, r, nw, w, silu_mul), h, residual,
+                       norm_weight, weight)
     normed, new_residual = torch_add_rmsnorm(h, residual, norm_weight, eps)
     y = F.linear(normed, weight)
     if silu_mul:
