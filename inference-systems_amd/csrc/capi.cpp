@@ -69,10 +69,10 @@ constexpr int64_t kDecodeMaxM = 32;
 
 // The plain GEMM also runs on splitk_decode up to M = 64 when W has fewer
 // than 65536 rows.  The table picks it there for narrow problems, where
-// mfma_staged's 64 x 64 tiles leave most CUs idle (bf16, M = 64: N = 1024,
-// K = 3584 6.5 against 15.5 us; N = 4096, K = 4096 10.0 against 19.0 us;
-// N = 8224, K = 1024 5.7 against 6.2 us), and not from 16384 rows or, above
-// 4096 rows, beyond K = 1024 (N = 12288, K = 2048: 14.3 against 11.6 us).
+// mfma_staged leaves CUs idle (bf16, M = 64, against its smallest tiles: N =
+// 1024, K = 3584 6.7 against 8.4 us; N = 2048, K = 2048 6.1 against 6.3 us; they
+// are level at N = 4096), and not from 16384 rows or, above 4096 rows, beyond
+// K = 1024 (N = 12288, K = 2048: 14.3 against 11.6 us).
 constexpr int64_t kSplitkPlainMaxM = 64;
 constexpr int64_t kSplitkPlainMaxRows = 65535;
 constexpr int64_t kSplitkPlainNarrowN = 4096;
@@ -398,15 +398,25 @@ bool gated_vector_ok(int64_t k, int64_t lda, int64_t ldg, int64_t group, int64_t
            group_stride % 8 == 0;
 }
 
-// The fused gate runs inside splitk_decode up to this M.  Every workgroup
-// gates all of A, so the sigmoids grow with M times the workgroup count; on
-// the Qwen3.5 o_proj (N = 1024, K = 2048) fused / gate kernel + GEMM measured
-// 4.7 / 5.4 us at M = 1, 6.1 / 6.6 us at M = 8, 9.9 / 7.0 us at M = 16.
+// The fused gate runs inside splitk_decode up to this M, and up to kDecodeMaxM
+// where workgroups of 8 rows of A and 16 W rows (32 above 2048 rows) still fit
+// the 256 CUs.  Every workgroup gates its rows of A again, which costs less
+// than a launch of its own up to 16384 sigmoids (fused against gate kernel +
+// GEMM, N = 1024, us, bf16): M = 8 / 16 / 32, K = 1024 4.7 / 4.9 / 5.0 against 5.6 /
+// 5.8 / 5.9; K = 2048 6.7 / 6.4 / 6.6 against 6.5 / 6.6 / 6.6; K = 4096 10.7 / 10.0 /
+// 10.2 against 8.1 / 8.2 / 8.3; M = 4, K = 4096, N = 1024 / 2560 8.4 / 10.5 against
+// 7.5 / 11.3.
 constexpr int64_t kGateFusedMaxM = 8;
+constexpr int64_t kGateFusedMaxWgs = 256;
+constexpr int64_t kGateFusedMaxWork = 16384;
 
 // The fused path copies whole 64-element lines of the gate, so a line must
 // not straddle two gate groups.
-bool gated_fused(int64_t m, int64_t group) { return m <= kGateFusedMaxM && group % 64 == 0; }
+bool gated_fused(int64_t m, int64_t n, int64_t k, int64_t group) {
+    if (group % 64 != 0 || m > kDecodeMaxM || (m < 8 ? m : 8) * k > kGateFusedMaxWork) return false;
+    const int64_t per = n <= 2048 ? 16 : 32;
+    return m <= kGateFusedMaxM || (n + per - 1) / per * ((m + 7) / 8) <= kGateFusedMaxWgs;
+}
 
 // Enough for any kernel that can run the problem (the fused gate uses none).
 int64_t gated_workspace_bytes(int64_t m, int64_t k) { return round_up_256(m * k * 2); }
@@ -426,7 +436,7 @@ int gated_entry(int forced_kernel, const void* a, const void* gate, const void* 
                          "gemm_gated needs 16-byte aligned a, gate and w with k, lda, ldg, group, group_stride "
                          "and ldw multiples of 8");
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool fused = forced_kernel < 0 ? gated_fused(m, group) : forced_kernel == NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
+    const bool fused = forced_kernel < 0 ? gated_fused(m, n, k, group) : forced_kernel == NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
     if (fused) {
         if (!(m <= kDecodeMaxM && group % 64 == 0))
             return set_error(NANOVLLM_GEMM_EUNSUPPORTED,
