@@ -57,6 +57,7 @@ SOURCES = [
     "gemm_direct.hip",
     "gemm_staged.hip",
     "gemm_wide.hip",
+    "gemm_mid.hip",
     "gemm_ragged.hip",
     "gemm_narrow.hip",
     "gemm_decode.hip",

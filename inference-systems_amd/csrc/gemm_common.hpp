@@ -461,6 +461,9 @@ int launch_mfma_narrow(const Problem& p, hipStream_t s);
 // mfma_staged's 256 x 256 tiles (gemm_wide.hip) and the grids that take them.
 bool mfma_wide_pays(const Problem& p);
 int launch_mfma_wide(const Problem& p, hipStream_t s);
+// mfma_staged's 128-row tiles for about one round (gemm_mid.hip) and the grids that take them.
+bool mfma_mid_pays(const Problem& p);
+int launch_mfma_mid(const Problem& p, hipStream_t s);
 int launch_splitk_decode(const Problem& p, hipStream_t s);
 int launch_gemv_decode(const Problem& p, hipStream_t s);
 

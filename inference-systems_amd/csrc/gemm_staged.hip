@@ -579,7 +579,10 @@ int launch_tile(const Problem& p, hipStream_t s) {
 //     40.0 -> 31.1 us against the burst schedule);
 //   * the greedy head, whose epilogue is written for 4 waves, takes the
 //     128 x 128 choices only;
-//   * large grids: the 256 x 256 tiles of gemm_wide.hip, by the rule there.
+//   * W[N,K] from K = 256: gemm_mid.hip's form of the 128 x 256 and 128 x 128
+//     tiles where its rule takes them, and on large grids the 256 x 256 tiles of
+//     gemm_wide.hip, by the rule there; the choices above are for the rest
+//     (B[K,N], shorter K, the LM head, SiLU pairs on 128 x 128).
 constexpr int64_t kSmallGridTiles = kCus / 2;
 template <int DT, int DT_OUT, int EPI, int RS = 0>
 int launch_epi(const Problem& p, hipStream_t s) {
@@ -632,6 +635,7 @@ int launch_typed(const Problem& p, hipStream_t s) {
 int launch_mfma_staged(const Problem& p, hipStream_t s) {
     if (mfma_wide_pays(p)) return launch_mfma_wide(p, s);
     if (mfma_narrow_pays(p)) return launch_mfma_narrow(p, s);
+    if (mfma_mid_pays(p)) return launch_mfma_mid(p, s);
     if (p.epi == EPI_ARGMAX) {
         constexpr int F = NANOVLLM_GEMM_F32;
         if (p.dtype_in == NANOVLLM_GEMM_BF16) return launch_epi<NANOVLLM_GEMM_BF16, F, EPI_ARGMAX>(p, s);

@@ -18,7 +18,7 @@
 //     every output has the bits mfma_staged's tiles give it;
 //   * within a group, the fragment of A the group has just used is reloaded
 //     for the next K-step, so the reads too are spread over the MFMAs.
-// Against the 128 x 256 and 128 x 128 tiles it took over from (bf16, inputs
+// Against the 128 x 256 and 128 x 128 tiles of mfma_staged (bf16, inputs
 // rotated): 4096^3 116.5 -> 91.6 us (1500 TFLOP/s), 8192^3 915 -> 717, 4096 x
 // 4096 x 1024 33.5 -> 28.4, 8192 x 8192 x 1024 129-139 -> 112, the fused
 // gate/up projection of 8192 x (2 x 3584) x 1024 129 -> 109 us.
@@ -335,18 +335,18 @@ int launch_typed(const Problem& p, hipStream_t s) {
 
 // Which grids take 256 x 256 tiles: those whose time on them, from a cost
 // model in units of 10 ns fitted to bf16 timings over M 512-8192, N 1024-12288
-// and K 256-4096 (kt K-tiles), is below that of mfma_staged's tiles:
+// and K 256-4096 (kt K-tiles), is below that of the 128-row tiles:
 //   * 256 x 256, one workgroup per CU: 8 + 1.25 kt us per full round of 256
 //     tiles, 4.5 + 0.9 kt us for a partial one plus up to 3.5 + 0.28 kt us as
 //     it fills (the chip clocks higher with CUs idle);
-//   * 128 x 256: 4 + 0.87 kt us for one round, then 3.4 + 0.86 kt us per 256
-//     tiles (two tiles' rounds overlap); 128 x 128 on a second round that is
-//     at most half full: 5.5 + 1.5 kt us.
-// Both sides measured (us, 128-row tiles against 256 x 256), K = 1024: 128
-// tiles of 256 x 256 17.4 / 22.2 (not taken), 144 28.5 / 21.9, 192 29.8 / 24.4,
-// 256 33.5 / 28.4, 288 44.0 / 47.0 (not taken), 384 49 / 49, 512 65.1 / 58.6,
-// 768 98 / 83, 1536 195 / 170; K = 256: 256 tiles 15.3 / 12.8, 576 31.0 / 32.5
-// (not taken), 768 46 / 37; K = 4096: 192 105 / 77, 256 118 / 93.
+//   * 128 x 256 (gemm_mid.hip): 1.6 us, 4.8 + 0.73 kt us per full round, 2.2 +
+//     0.48 kt us for a partial one plus up to 1.2 + 0.27 kt us as it fills; or 4 +
+//     1.08 kt us on 128 x 128 tiles where those are at most 512, two to each CU.
+// Both sides measured (us, 128-row tiles against 256 x 256), K = 1024: 272 tiles
+// of 128 x 256 28.6 / 25.3, 320 28.5 / 25.7, 416 31.5 / 28.9, 896 (SiLU pairs) 66.0 /
+// 59.4, 1579 x 4992 (260, and 507 of 128 x 128) 21.6 / 24.6 (not taken), 576 44.4 /
+// 50.2 and 768 49.4 / 53.5 (not taken); K = 512: 416 20.4 / 19.2, 768 31.9 / 34.3
+// (not taken); K = 3072: 272 68.2 / 59.7, 576 109 / 123 (not taken).
 bool mfma_wide_pays(const Problem& p) {
     if (p.b_layout != NANOVLLM_GEMM_B_NK || p.k < 256 || p.k > (int64_t(1) << 30)) return false;
     if (p.epi != EPI_NONE && p.epi != EPI_SILU_MUL) return false;
@@ -364,7 +364,11 @@ bool mfma_wide_pays(const Problem& p) {
     const int64_t rest = wide % kCus;
     const int64_t wide_cost =
         wide / kCus * (800 + 125 * kt) + (rest > 0 ? 450 + 90 * kt + rest * (350 + 28 * kt) / kCus : 0);
-    const int64_t narrow_cost = narrow <= 3 * kCus / 2 ? 550 + 150 * kt : narrow * (340 + 86 * kt) / kCus;
+    const int64_t tiles128 = (p.m + 127) / 128 * ((cols + 127) / 128);
+    const int64_t part = narrow % kCus;
+    int64_t narrow_cost =
+        160 + narrow / kCus * (480 + 73 * kt) + (part > 0 ? 220 + 48 * kt + part * (120 + 27 * kt) / kCus : 0);
+    if (tiles128 <= 2 * kCus && 400 + 108 * kt < narrow_cost) narrow_cost = 400 + 108 * kt;
     return wide_cost < narrow_cost;
 }
 
