@@ -318,12 +318,14 @@ __device__ __forceinline__ float norm_scale(float ss, int64_t k, float eps) {
 // 0xFFFFFFFF - column in the low word, so the largest key is the largest
 // logit and, among equal logits, the first column (torch.argmax's rule).
 // Key 0 is below every real key.
-__device__ __forceinline__ uint64_t argmax_key(float v, int64_t col) {
+__device__ __forceinline__ uint32_t argmax_order(float v) {
     // -0 ranks equal to +0, and every NaN ranks above every number (as in
     // torch.argmax): both are canonicalised first.
     const uint32_t b = v != v ? 0x7FC00000u : (v == 0.0f ? 0u : __builtin_bit_cast(uint32_t, v));
-    const uint32_t ordered = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-    return (uint64_t(ordered) << 32) | uint64_t(0xFFFFFFFFu - uint32_t(col));
+    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ uint64_t argmax_key(float v, int64_t col) {
+    return (uint64_t(argmax_order(v)) << 32) | uint64_t(0xFFFFFFFFu - uint32_t(col));
 }
 
 // Sampled LM head (EPI_ARGMAX with a temperature per row).  Sampler

@@ -468,33 +468,43 @@ __global__ __launch_bounds__(WGM * WGN * 64) void mfma_staged_kernel(
     }
     __syncthreads();
     if constexpr (EPI == EPI_ARGMAX) {
-        // Greedy LM head: per row of the tile, the best of its BN columns
-        // (two threads per row, 64 columns each), one key per row.
-        static_assert(OB == 4 && NT == 2 * BM, "fp32 tile, two threads per row");
-        const int r = tid >> 1, h = tid & 1;
-        const float* rowp = reinterpret_cast<const float*>(ctile + r * PITCH);
-        uint64_t best = 0;
+        // LM head: per row of the tile, the best of its BN columns, TPR threads
+        // per row.  A thread takes groups of 4 adjacent columns (one noise draw
+        // serves 4 scores on a sampled row: n0 is a multiple of BN), group S h +
+        // i % S + 16 (i / S) in step i, which puts the 16 lanes the LDS serves
+        // at once on 16 distinct bank groups.  The columns ascend, so keeping
+        // the first of equal values keeps the first index.
+        constexpr int TPR = NT / BM, S = 16 / TPR;
+        static_assert(OB == 4 && (TPR == 2 || TPR == 4) && BN % 64 == 0, "fp32 tile, whole steps");
+        const int r = tid / TPR, h = tid % TPR;
+        const char* rowp = ctile + r * PITCH;
+        uint32_t best_ord = 0;   // below every value's
+        int best_col = 0;
         if (m0 + r < m) {
-            // Groups of 4 adjacent columns: one noise draw serves 4 scores on
-            // a sampled row (n0 is a multiple of BN).
             const float t = sample_temperature(m0 + r, sa);
-            for (int c4 = 0; c4 < BN / 2; c4 += 4) {
-                const int col0 = h * (BN / 2) + c4;
-                if (n0 + col0 >= n) break;
+            for (int i = 0; i < BN / 4 / TPR; ++i) {
+                const int col0 = 4 * (S * h + i % S + 16 * (i / S));
+                if (n0 + col0 >= n) continue;
+                const f32x4_t v4 = *reinterpret_cast<const f32x4_t*>(rowp + 4 * col0);
                 const u32x4_t x = t != 0.0f ? sample_words(m0 + r, (n0 + col0) >> 2, sa) : u32x4_t{0u, 0u, 0u, 0u};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const int col = col0 + j;
-                    if (n0 + col >= n) break;
-                    const float v = ranked_logit(rowp[col], sa);
-                    const uint64_t key = argmax_key(t != 0.0f ? gumbel_score(v, t, x[j]) : v, n0 + col);
-                    best = key > best ? key : best;
+                    const float v = ranked_logit(v4[j], sa);
+                    const uint32_t ord = argmax_order(t != 0.0f ? gumbel_score(v, t, x[j]) : v);
+                    if (n0 + col0 + j < n && ord > best_ord) {
+                        best_ord = ord;
+                        best_col = col0 + j;
+                    }
                 }
             }
         }
-        const uint64_t other = (uint64_t(uint32_t(__shfl_xor(int(best >> 32), 1))) << 32) |
-                               uint64_t(uint32_t(__shfl_xor(int(best & 0xFFFFFFFFu), 1)));
-        best = other > best ? other : best;
+        uint64_t best = best_ord == 0 ? 0 : (uint64_t(best_ord) << 32) | uint64_t(0xFFFFFFFFu - uint32_t(n0 + best_col));
+#pragma unroll
+        for (int off = TPR / 2; off >= 1; off >>= 1) {
+            const uint64_t other = (uint64_t(uint32_t(__shfl_xor(int(best >> 32), off))) << 32) |
+                                   uint64_t(uint32_t(__shfl_xor(int(best & 0xFFFFFFFFu), off)));
+            best = other > best ? other : best;
+        }
         if (h == 0 && m0 + r < m) keys[(m0 + r) * int64_t(tiles_n) + tn] = best;
         return;
     }
@@ -577,8 +587,10 @@ int launch_tile(const Problem& p, hipStream_t s) {
 //   * otherwise (128 < tiles <= 256): 128 x 128, 4 waves, 3-deep ring,
 //     spread copies, one workgroup per CU (4096 x 1024 x 3584, 256 tiles:
 //     40.0 -> 31.1 us against the burst schedule);
-//   * the greedy head, whose epilogue is written for 4 waves, takes the
-//     128 x 128 choices only;
+//   * the LM head: as above, but sampled at M <= 128 on more than one round of
+//     128 x 256 tiles stays on 128 x 128, whose two workgroups to a CU hide the
+//     scores' arithmetic better (151936 x 1024, M = 128: 104 against 118 us; M = 300
+//     235 / 221, greedy 208 / 173; 60000 x 768, M = 128 37 / 33);
 //   * W[N,K] from K = 256: gemm_mid.hip's form of the 128 x 256 and 128 x 128
 //     tiles where its rule takes them, and on large grids the 256 x 256 tiles of
 //     gemm_wide.hip, by the rule there; the choices above are for the rest
@@ -591,11 +603,10 @@ int launch_epi(const Problem& p, hipStream_t s) {
     const int64_t tiles = ((p.m + 127) / 128) * ((n_tiles + 127) / 128);
     if constexpr (EPI == EPI_NONE)
         if (tiles <= kSmallGridTiles) return launch_tile<DT, DT_OUT, 64, 64, 2, 2, 3, EPI, RS, 1>(p, s);
-    if constexpr (EPI != EPI_ARGMAX) {
-        const int64_t wide = ((p.m + 127) / 128) * ((n_tiles + 255) / 256);
-        if (wide > kCus / 2 && (wide <= kCus || wide > 3 * kCus / 2))
-            return launch_tile<DT, DT_OUT, 128, 256, 2, 4, 3, EPI, RS, 1>(p, s);
-    }
+    const int64_t wide = ((p.m + 127) / 128) * ((n_tiles + 255) / 256);
+    const bool head_loses = EPI == EPI_ARGMAX && p.sample.temperature != nullptr && wide > kCus && p.m <= 128;
+    if (wide > kCus / 2 && (wide <= kCus || wide > 3 * kCus / 2) && !head_loses)
+        return launch_tile<DT, DT_OUT, 128, 256, 2, 4, 3, EPI, RS, 1>(p, s);
     if (tiles <= kCus) return launch_tile<DT, DT_OUT, 128, 128, 2, 2, 3, EPI, RS, 1>(p, s);
     return launch_tile<DT, DT_OUT, 128, 128, 2, 2, 2, EPI, RS, 0>(p, s);
 }
