@@ -446,6 +446,44 @@ __device__ __forceinline__ void grouped_tile(int t, int tiles_m, int tiles_n, in
 }
 
 // ---------------------------------------------------------------------------
+// A C tile of ROWS x COLS elements of OB bytes from LDS (row pitch `pitch`
+// bytes) to rows of C that are not 16-byte aligned; the tile's first `rows` rows
+// and `cols` columns exist.  Adjacent lanes store adjacent words, or elements
+// where rows are not 4-byte aligned either: a chunk of 8 elements per lane costs
+// an instruction for each, every one over 8 cache lines (bf16, 1100 x 2500 x 1024
+// 15.4 -> 11.7 us).
+// ---------------------------------------------------------------------------
+template <int OB, int ROWS, int COLS, int NT>
+__device__ __forceinline__ void store_unaligned(const char* ctile, int pitch, char* c, int64_t ldc, int64_t rows,
+                                                int64_t cols, int tid) {
+    const int nr = rows < ROWS ? int(rows) : ROWS, nc = cols < COLS ? int(cols) : COLS;
+    if (OB == 4 || (reinterpret_cast<uintptr_t>(c) % 4 == 0 && ldc % 2 == 0)) {
+        constexpr int WPR = COLS * OB / 4;
+        const int words = nc * OB / 4;
+#pragma unroll 4
+        for (int e = tid; e < ROWS * WPR; e += NT) {
+            const int r = e / WPR, w = e % WPR;
+            if (r < nr && w < words)
+                *reinterpret_cast<uint32_t*>(c + int64_t(r) * ldc * OB + 4 * w) =
+                    *reinterpret_cast<const uint32_t*>(ctile + r * pitch + 4 * w);
+        }
+        if (OB == 2 && (nc & 1)) {
+            for (int r = tid; r < nr; r += NT)
+                *reinterpret_cast<uint16_t*>(c + (int64_t(r) * ldc + nc - 1) * OB) =
+                    *reinterpret_cast<const uint16_t*>(ctile + r * pitch + (nc - 1) * OB);
+        }
+        return;
+    }
+#pragma unroll 4
+    for (int e = tid; e < ROWS * COLS; e += NT) {
+        const int r = e / COLS, col = e % COLS;
+        if (r < nr && col < nc)
+            *reinterpret_cast<uint16_t*>(c + (int64_t(r) * ldc + col) * OB) =
+                *reinterpret_cast<const uint16_t*>(ctile + r * pitch + col * OB);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Launchers (one per kernel family).  Each returns NANOVLLM_GEMM_OK or a
 // negative code; the caller has already validated the problem and checked
 // that the kernel supports it.

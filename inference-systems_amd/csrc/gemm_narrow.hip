@@ -208,6 +208,11 @@ __global__ __launch_bounds__(WGM * WGN * 64) void mfma_narrow_kernel(
         }
     }
     __syncthreads();
+    if (!c_vec) {
+        store_unaligned<OB, BM, BNO, NT>(ctile, PITCH, static_cast<char*>(c) + (m0 * ldc + n0) * OB, ldc, m - m0, n - n0,
+                                         tid);
+        return;
+    }
 #pragma unroll 2
     for (int e = tid; e < BM * CPR; e += NT) {
         const int r = e / CPR, chunk = e % CPR;
@@ -215,7 +220,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) void mfma_narrow_kernel(
         if (grow >= m || gcol >= n) continue;
         const u32x4_t val = *reinterpret_cast<const u32x4_t*>(ctile + r * PITCH + chunk * 16);
         char* gdst = static_cast<char*>(c) + (grow * ldc + gcol) * OB;
-        if (c_vec && gcol + EPC <= n) {
+        if (gcol + EPC <= n) {
             __builtin_nontemporal_store(val, reinterpret_cast<u32x4_t*>(gdst));
         } else {
             const int valid = int(min_i64(EPC, n - gcol));

@@ -523,13 +523,18 @@ __global__ __launch_bounds__(WGM * WGN * 64) void mfma_staged_kernel(
         }
         return;
     }
+    if (!c_vec) {
+        store_unaligned<OB, BM, BNO, NT>(ctile, PITCH, static_cast<char*>(c) + (m0 * ldc + n0) * OB, ldc, m - m0, n - n0,
+                                         tid);
+        return;
+    }
     for (int r = tid / CPR; r < BM; r += ROWS_PER_PASS) {
         const int64_t grow = m0 + r;
         const int64_t gcol = n0 + chunk * EPC;
         if (grow >= m || gcol >= n) continue;
         const u32x4_t val = *reinterpret_cast<const u32x4_t*>(ctile + r * PITCH + chunk * 16);
         char* gdst = static_cast<char*>(c) + (grow * ldc + gcol) * OB;
-        if (c_vec && gcol + EPC <= n) {
+        if (gcol + EPC <= n) {
             __builtin_nontemporal_store(val, reinterpret_cast<u32x4_t*>(gdst));
         } else {
             const int valid = int(min_i64(EPC, n - gcol));
