@@ -310,12 +310,13 @@ int nanovllm_gemm_sample_with_kernel(int kernel_id,
  * (qwen3_5.py:81-86): element (i, k) at
  *     gate[i * ldg + (k / group) * group_stride + k % group]
  * (group = head_dim, group_stride = 2 head_dim for q_gate; a contiguous
- * [m, k] gate is group = group_stride = k).  For m <= 8 and group a
- * multiple of 64 the gate is applied inside the split-K decode kernel (one
- * launch, no workspace; every workgroup gates all of A, which stops paying
- * above m = 8); otherwise a gate kernel writes the gated operand to the
- * workspace (nanovllm_gemm_gated_workspace_bytes() bytes) and the GEMM the
- * selection table picks reads it.  Inputs f16 or bf16, output the input
+ * [m, k] gate is group = group_stride = k).  For group a multiple of 64 and
+ * m <= 8, or m <= 32 on narrow w, the gate is applied inside the split-K decode
+ * kernel (one launch, no workspace) while its workgroups, each of which gates
+ * its rows of A, have little to gate; otherwise a gate kernel writes the gated
+ * operand to the workspace (nanovllm_gemm_gated_workspace_bytes() bytes) and
+ * the GEMM the selection table picks reads it.  With m <= 8 and no workspace
+ * the fused form runs at any k.  Inputs f16 or bf16, output the input
  * type or f32, on the vector path (16-byte aligned a, gate and w; k, lda,
  * ldg, group, group_stride and ldw multiples of 8).  Asynchronous, no
  * allocation, capturable. */
@@ -328,8 +329,8 @@ int nanovllm_gemm_gated(const void* a, const void* gate, const void* w, void* c,
                         void* stream);
 
 /* Workspace bytes nanovllm_gemm_gated needs with any kernel that can run
- * the problem (the fused gate uses none: workspace may then be null), or a
- * negative code.  Pure host function. */
+ * the problem (the fused gate uses none: for m <= 8 and group a multiple of 64
+ * workspace may be null), or a negative code.  Pure host function. */
 int64_t nanovllm_gemm_gated_workspace_bytes(int64_t m, int64_t k, int64_t group, int dtype_in);
 
 /* The gated GEMM forced onto one kernel: splitk_decode runs the fused gate

@@ -436,7 +436,13 @@ int gated_entry(int forced_kernel, const void* a, const void* gate, const void* 
                          "gemm_gated needs 16-byte aligned a, gate and w with k, lda, ldg, group, group_stride "
                          "and ldw multiples of 8");
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool fused = forced_kernel < 0 ? gated_fused(m, n, k, group) : forced_kernel == NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
+    const int64_t need = round_up_256(m * k * 2);
+    const bool have_ws = workspace != nullptr && workspace_bytes >= need && aligned16_ptr(workspace);
+    // Up to kGateFusedMaxM a caller may leave the workspace out: the fused gate
+    // then runs whatever it costs.
+    const bool fused = forced_kernel < 0
+                           ? gated_fused(m, n, k, group) || (!have_ws && m <= kGateFusedMaxM && group % 64 == 0)
+                           : forced_kernel == NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
     if (fused) {
         if (!(m <= kDecodeMaxM && group % 64 == 0))
             return set_error(NANOVLLM_GEMM_EUNSUPPORTED,
@@ -452,8 +458,7 @@ int gated_entry(int forced_kernel, const void* a, const void* gate, const void* 
     }
     // The gated operand goes to the workspace (leading dimension k), then the
     // GEMM the table (or the caller) picks for it.
-    const int64_t need = round_up_256(m * k * 2);
-    if (workspace == nullptr || workspace_bytes < need || !aligned16_ptr(workspace))
+    if (!have_ws)
         return set_error(NANOVLLM_GEMM_EINVAL,
                          "this problem needs a 16-byte aligned workspace of %lld bytes (got %lld)", (long long)need,
                          (long long)workspace_bytes);

@@ -85,3 +85,20 @@ def test_gate_kernel_group_placement():
     want = (a.double() * sg).reshape(m, -1)
     # two roundings to bf16, of the sigmoid and of the product: 2^-8 each
     assert bool(((got.double() - want).abs() <= want.abs() * (2 ** -7 + 2 ** -12)).all())
+
+
+@pytest.mark.parametrize("k", [1024, 4096])
+def test_gate_without_workspace(k):
+    """Up to 8 rows the C ABI takes no workspace: the fused gate runs, at any K,
+    with the bits of the path that has one."""
+    m, n = 8, 520
+    gen = torch.Generator().manual_seed(k)
+    a = torch.randn((m, k // 64, 64), generator=gen).bfloat16().to(DEV)
+    gate = torch.randn((m, k // 64, 64), generator=gen).bfloat16().to(DEV)
+    w = (torch.randn((n, k), generator=gen) * 0.05).bfloat16().to(DEV)
+    out = torch.empty((m, n), dtype=BF16, device=DEV)
+    L.gated_raw(a.data_ptr(), gate.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, k, k, 64, 64, k, n, L.BF16, L.BF16,
+                None, 0, torch.cuda.current_stream().cuda_stream)
+    want = K.gemm_gated(a, gate, w)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
