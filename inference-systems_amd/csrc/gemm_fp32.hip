@@ -227,10 +227,10 @@ __global__ __launch_bounds__(kT32Threads) void fp32_tiled_kernel(
 //   * MFMA step s of a K-tile takes k = STEPS (l / LH) + s in lane l, LH the
 //     lanes per k group of the instruction, so a lane's A (and W[N,K])
 //     values of a K-tile are one run of contiguous floats (ds_read_b128).
-// Configurations by grid size (fp32, W[N,K] unless noted, us).  The first three
-// run v_mfma_f32_16x16x4_f32 with K split over two wave groups (BK = 64): a
-// wave then has half the MFMA chain of a K-tile, and the two partial sums come
-// closer to the exact one (relative error at K = 1024 4.1e-7 against 5.7e-7 of
+// Configurations by grid size (fp32, W[N,K] unless noted, us).  All but the last
+// run v_mfma_f32_16x16x4_f32, with K split over two wave groups (and K-tiles of
+// 64, unless noted): a wave then has half the MFMA chain of a K-tile, and the two
+// partial sums come closer to the exact one (relative error at K = 1024 4.1e-7 against 5.7e-7 of
 // one chain).  Fewer than 512 tiles of 64 x 64 leave CUs idle or bound by the
 // chain of MFMAs over rows past M, so tiles are as small as two workgroups to a
 // CU allow; against the 64 x 32 tiles that took all of these grids before:
@@ -239,11 +239,15 @@ __global__ __launch_bounds__(kT32Threads) void fp32_tiled_kernel(
 //     8128 138 -> 98, 64 x 4096 x 1024 12.6 -> 8.4;
 //   * 32 x 32, up to 512: 200 x 2048 x 1024 13.0 -> 12.0 (16 x 32 12.7), 512 x
 //     1024 x 1024 12.4 -> 11.6 (32 x 64 11.9);
-//   * 32 x 64: 1024^3 19.8 -> 19.2, B[K,N] 21.7 -> 20.9, 300 x 4096 x 1024 28.9 ->
-//     28.3;
-//   * from 512 tiles of 64 x 64: 64 x 64 tiles, v_mfma_f32_32x32x2_f32 in two accumulator chains (odd
-//     steps in the second, added before the store), BK = 32, on larger grids
-//     (2048^3 156.7 -> 126.6 us, 4096^3 1208.6 -> 966.6 us).
+//   * 32 x 64 or 64 x 64 on K-tiles of 32, whichever puts less on the busiest
+//     CU: 900 x 1100 x 1500 (522 / 270 workgroups) 42.3 -> 37.8 (64 x 64 48.1), 300 x
+//     4096 x 1024 29.5 -> 26.3 (33.0), 1400 x 1300 x 512 (924 / 462) 22.2 -> 20.4
+//     (32 x 64 23.9), 1024^3 21.0 -> 20.2.  B[K,N] reads its fragments a float
+//     at a time, so there 64 x 32 with one chain stays instead of 64 x 64 (1024^3
+//     19.7 against 20.1, 222 x 3648 x 960 20.4 / 20.8);
+//   * from 512 tiles of 64 x 64: those, v_mfma_f32_32x32x2_f32 in two accumulator
+//     chains (odd steps in the second, added before the store), BK = 32 (2048^3
+//     156.7 -> 126.6 us, 4096^3 1208.6 -> 966.6 us).
 // Measured beside the last: 64 x 64 tiles with one chain, BK = 32, 20.6 / 148.4
 // / 959.6 us; 32 x 32 tiles, BK = 64, 19.2-20.8 / 143 / 1107 us; one
 // K-tile of loads in flight more or less, half a K-tile of MFMAs after the
@@ -585,10 +589,15 @@ void launch_buffered(const Problem& p, hipStream_t s) {
 template <int BL>
 void launch_buffered_for(const Problem& p, hipStream_t s) {
     const int64_t tiles64 = ((p.m + 63) / 64) * ((p.n + 63) / 64);
+    const auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };   // on the busiest CU
     const auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
     if (tiles(16, 32) <= 512) launch_buffered<BL, 16, 32, 64, 16, 1, 2>(p, s);
     else if (tiles(32, 32) <= 512) launch_buffered<BL, 32, 32, 64, 16, 1, 2>(p, s);
-    else if (tiles64 < 512) launch_buffered<BL, 32, 64, 64, 16, 1, 2>(p, s);
+    else if (tiles64 < 512 && 2 * rounds(tiles64) <= rounds(tiles(32, 64))) {
+        if constexpr (BL == NANOVLLM_GEMM_B_KN) launch_buffered<BL, 64, 32, 64, 16, 1>(p, s);
+        else launch_buffered<BL, 64, 64, 32, 16, 1, 2>(p, s);
+    }
+    else if (tiles64 < 512) launch_buffered<BL, 32, 64, 32, 16, 1, 2>(p, s);
     else launch_buffered<BL, 64, 64, 32, 32, 2>(p, s);
 }
 
