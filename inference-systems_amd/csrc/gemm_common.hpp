@@ -216,35 +216,20 @@ __device__ __forceinline__ u32x4_t load16(const void* p) {
     return *static_cast<const u32x4_t*>(p);
 }
 
-// x * sigmoid(x) = x / (1 + e^-x) in fp32, from the hardware base-2
-// exponential and reciprocal with the roundings that matter put back:
-//   * e^-x = 2^h (1 + l ln 2), where h = round(-x log2 e) and l is the rest
-//     of the product (the fma's exact remainder and the low part of log2 e),
-//     so the exponent's rounding does not grow with |x|;
-//   * the quotient takes one residual step, which carries the l part of the
-//     denominator too, and v_div_fixup settles infinite operands (x below
-//     -88.7: -0; +inf: +inf) and NaN.  Numerator and denominator carry a
-//     factor 1/4, so the reciprocal stays normal up to the largest finite
-//     denominator.
-// The median and minimum keep l (NaN at x = +-inf) and the correction's
-// factor (inf below -88.7) finite.  A fused gate/up epilogue runs this once
-// per output on the VALU while the matrix cores wait: 17 instructions against
-// ~55 for the library exp and the IEEE divide.
+// x * sigmoid(x) = x / (1 + e^-x) in fp32: the library's exponential and the
+// correctly rounded quotient, with the bits of `x / (1.0f + expf(-x))` for every
+// fp32 x.  The compiler's IEEE divide spends 10 instructions on operands of any
+// size; the denominator here is at least 1, so one residual step on the hardware
+// reciprocal rounds every quotient there is correctly (compared over all 2^32 x).
+// The reciprocal is taken of a quarter of the denominator, which keeps it normal
+// up to the largest finite one, and v_div_fixup settles infinite operands (-0
+// below -88.7, NaN at -inf, +inf at +inf) and NaN.  A fused gate/up epilogue runs
+// this once per output on the VALU while the matrix cores wait.
 __device__ __forceinline__ float silu_f32(float x) {
-    constexpr float kLog2eHi = 1.44269502162933349609f;    // log2 e rounded to fp32
-    constexpr float kLog2eLo = 1.92596299112661746888e-8f; // log2 e - kLog2eHi
-    constexpr float kLn2 = 0.693147180559945309f;
-    const float h = -x * kLog2eHi;
-    const float rest = __builtin_fmaf(-x, kLog2eLo, __builtin_fmaf(-x, kLog2eHi, -h));
-    const float l = __builtin_amdgcn_fmed3f(rest, -1e-4f, 1e-4f);   // |l| < 2e-5 for finite 2^h
-    const float q4 = 0.25f * __builtin_amdgcn_exp2f(h);
-    const float d = 0.25f + q4;
-    const float dl = __builtin_fminf(q4, 0x1p126f) * (l * kLn2);
-    const float n = 0.25f * x;
-    const float r = __builtin_amdgcn_rcpf(d);
-    const float q = n * r;
-    const float res = __builtin_fmaf(-dl, q, __builtin_fmaf(-d, q, n));
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(res, r, q), d, n);
+    const float d = 1.0f + expf(-x);
+    const float r = 0.25f * __builtin_amdgcn_rcpf(0.25f * d);
+    const float q = x * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
 }
 
 // sigmoid(x) = 1 / (1 + 2^(-x log2 e)) with the hardware base-2 exponential
