@@ -248,6 +248,10 @@ __global__ __launch_bounds__(kThreads) void mfma_wide_kernel(
     static_assert(EP_ROWS % ROWS_PER_PASS == 0, "copy passes");
     char* ctile = reinterpret_cast<char*>(ring);
     const int chunk = tid % CPR;
+    // The row scales from a scalar base and 32-bit rows: 64-bit row numbers are
+    // kept through the K loop, which has no register left for them.
+    const float* scale = RS ? row_scale + m0 : nullptr;
+    const int last_row = static_cast<int>(min_i64(kBM, m - m0)) - 1;
 #pragma unroll 1
     for (int ep = 0; ep < EPASS; ++ep) {
         __syncthreads();
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(kThreads) void mfma_wide_kernel(
             for (int i = 0; i < kMI; ++i) {
                 const int row = wm * kWM + 16 * i + r16;
                 float rs = 1.0f;
-                if constexpr (RS) rs = row_scale[min_i64(m0 + row, m - 1)];
+                if constexpr (RS) rs = scale[row < last_row ? row : last_row];
                 char* rowp = ctile + (row - ep * EP_ROWS) * PITCH;
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
