@@ -316,10 +316,11 @@ int nanovllm_gemm_sample_with_kernel(int kernel_id,
  * its rows of A, have little to gate; otherwise a gate kernel writes the gated
  * operand to the workspace (nanovllm_gemm_gated_workspace_bytes() bytes) and
  * the GEMM the selection table picks reads it.  With m <= 8 and no workspace
- * the fused form runs at any k.  Inputs f16 or bf16, output the input
- * type or f32, on the vector path (16-byte aligned a, gate and w; k, lda,
- * ldg, group, group_stride and ldw multiples of 8).  Asynchronous, no
- * allocation, capturable. */
+ * the fused form runs at any k; above m = 8 the workspace is required
+ * whichever form runs.  Inputs f16 or bf16, output the input type or f32, on
+ * the vector path (16-byte aligned a, gate and w; k, lda, ldg, group,
+ * group_stride and ldw multiples of 8).  Asynchronous, no allocation,
+ * capturable. */
 int nanovllm_gemm_gated(const void* a, const void* gate, const void* w, void* c,
                         int64_t m, int64_t n, int64_t k,
                         int64_t lda, int64_t ldg, int64_t group, int64_t group_stride,

@@ -439,10 +439,10 @@ int gated_entry(int forced_kernel, const void* a, const void* gate, const void* 
     const int64_t need = round_up_256(m * k * 2);
     const bool have_ws = workspace != nullptr && workspace_bytes >= need && aligned16_ptr(workspace);
     // Up to kGateFusedMaxM a caller may leave the workspace out: the fused gate
-    // then runs whatever it costs.
-    const bool fused = forced_kernel < 0
-                           ? gated_fused(m, n, k, group) || (!have_ws && m <= kGateFusedMaxM && group % 64 == 0)
-                           : forced_kernel == NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
+    // then runs whatever it costs.  Above, the workspace is asked for whichever
+    // form runs, so a call that leaves it out is refused at every n alike.
+    const bool fused = forced_kernel < 0 ? (have_ws ? gated_fused(m, n, k, group) : m <= kGateFusedMaxM && group % 64 == 0)
+                                         : forced_kernel == NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
     if (fused) {
         if (!(m <= kDecodeMaxM && group % 64 == 0))
             return set_error(NANOVLLM_GEMM_EUNSUPPORTED,

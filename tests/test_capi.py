@@ -368,6 +368,12 @@ def test_gated_validates_before_launch(lib):
     # M > 32 needs the workspace
     rc = call(d, d, d, d, 40, 64, 512, 512, 1024, 256, 512, 512, 64, BF16, BF16, None, 0, None)
     assert rc == L.EINVAL and "workspace" in L.last_error()
+    # and so does M > 8 where the fused form, which uses none, would run: too
+    # small, unaligned or absent is refused whatever N
+    for m, n in ((9, 64), (16, 1024), (32, 1024)):
+        for ws, size in ((None, 0), (d, m * 512 * 2 - 1), (d + 2, m * 512 * 2 + 256)):
+            rc = call(d, d, d, d, m, n, 512, 512, 1024, 256, 512, 512, n, BF16, BF16, ws, size, None)
+            assert rc == L.EINVAL and "workspace" in L.last_error()
     # the fused gate cannot take a head size that is not a multiple of 64
     rc = lib.nanovllm_gemm_gated_with_kernel(L.KERNEL_SPLITK_DECODE, d, d, d, d, 4, 64, 480, 480, 960, 40, 80, 480,
                                              64, BF16, BF16, None, 0, None)
