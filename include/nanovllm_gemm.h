@@ -406,6 +406,12 @@ const char* nanovllm_gemm_kernel_name(int kernel_id);
 /* Message describing the last error on the calling thread ("" if none). */
 const char* nanovllm_gemm_last_error(void);
 
+/* Kernel and tile (rows of a x columns of c per workgroup) that the last GEMM
+ * call on the calling thread launched, e.g. "mfma_narrow 32x64" ("" if none);
+ * valid until the thread's next call of this function.  For tests and
+ * profiles. */
+const char* nanovllm_gemm_last_kernel(void);
+
 /* Library version, (major << 16) | minor. */
 int nanovllm_gemm_version(void);
 

@@ -67,6 +67,7 @@ SIGNATURES = {
                                               + [_INT, _INT, _INT, _VP, _I64, _VP]),
     "nanovllm_gemm_kernel_name": (ctypes.c_char_p, [_INT]),
     "nanovllm_gemm_last_error": (ctypes.c_char_p, []),
+    "nanovllm_gemm_last_kernel": (ctypes.c_char_p, []),
     "nanovllm_gemm_version": (_INT, []),
 }
 
@@ -120,6 +121,11 @@ def is_available() -> bool:
 
 def last_error() -> str:
     return load().nanovllm_gemm_last_error().decode()
+
+
+def last_kernel() -> str:
+    """Kernel and tile the last GEMM call on this thread launched ("mfma_narrow 32x64")."""
+    return load().nanovllm_gemm_last_kernel().decode()
 
 
 def kernel_name(kernel_id: int) -> str:

@@ -14,6 +14,9 @@ namespace nvg {
 namespace {
 thread_local std::string g_last_error;
 
+struct LaunchedKernel { const char* name; int rows, cols; };
+thread_local LaunchedKernel g_last_kernel = {nullptr, 0, 0};
+
 bool dtype_pair_ok(int din, int dout) {
     switch (din) {
         case NANOVLLM_GEMM_F32: return dout == NANOVLLM_GEMM_F32;
@@ -572,9 +575,10 @@ int set_error(int code, const char* fmt, ...) {
     return code;
 }
 
-int check_launch(const char* kernel) {
+int check_launch(const char* kernel, int rows, int cols) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(NANOVLLM_GEMM_ELAUNCH, "%s launch failed: %s", kernel, hipGetErrorString(e));
+    if (rows > 0) g_last_kernel = {kernel, rows, cols};
     return NANOVLLM_GEMM_OK;
 }
 
@@ -806,6 +810,14 @@ int nanovllm_gemm_add_rmsnorm_with_kernel(int kernel_id, const void* h, const vo
 }
 
 const char* nanovllm_gemm_last_error(void) { return nvg::g_last_error.c_str(); }
+
+const char* nanovllm_gemm_last_kernel(void) {
+    thread_local char text[64];
+    const nvg::LaunchedKernel& k = nvg::g_last_kernel;
+    if (k.name == nullptr) return "";
+    snprintf(text, sizeof text, "%s %dx%d", k.name, k.rows, k.cols);
+    return text;
+}
 
 int nanovllm_gemm_version(void) { return (2 << 16) | 0; }
 

@@ -555,7 +555,7 @@ int launch_cfg(const Problem& p, hipStream_t s) {
                        grid, block, 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.c, p.m, p.n, p.k,
                        p.lda, p.ldb, p.ldc, p.keys, pro, p.sample);
-    return check_launch("splitk_decode");
+    return check_launch("splitk_decode", AROWS, 16 * OG);
 }
 
 }  // namespace

@@ -24,7 +24,7 @@ namespace nvg {
 
 int set_error(int code, const char*, ...) { return code; }
 
-int check_launch(const char*) {
+int check_launch(const char*, int, int) {
     return hipGetLastError() == hipSuccess ? NANOVLLM_GEMM_OK : NANOVLLM_GEMM_ELAUNCH;
 }
 

@@ -514,7 +514,9 @@ int argmax_scratch(hipStream_t stream, void** ptr);
 // Records a message for nanovllm_gemm_last_error() and returns `code`.
 int set_error(int code, const char* fmt, ...);
 
-// Converts a hipError_t after a launch into a return code.
-int check_launch(const char* kernel);
+// Converts a hipError_t after a launch into a return code, and notes a GEMM
+// kernel's name and tile (rows of A x columns of C; 0 x 0: not a GEMM kernel)
+// for nanovllm_gemm_last_kernel().
+int check_launch(const char* kernel, int rows = 0, int cols = 0);
 
 }  // namespace nvg

@@ -143,7 +143,7 @@ int launch_typed(const Problem& p, hipStream_t s) {
             hipLaunchKernelGGL((mfma_direct_kernel<DT, DT_OUT, NANOVLLM_GEMM_B_KN, 0>), grid, block, 0, s, a, b, p.c,
                                p.m, p.n, p.k, p.lda, p.ldb, p.ldc, ti, tj, vec_a, vec_b);
     }
-    return check_launch("mfma_direct");
+    return check_launch("mfma_direct", 64, 64);
 }
 
 // Every row of A and B starts and ends on a 16-byte chunk: the problems

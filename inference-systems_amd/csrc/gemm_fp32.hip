@@ -573,32 +573,31 @@ int launch_fp32_naive(const Problem& p, hipStream_t s) {
     else
         hipLaunchKernelGGL(fp32_naive_kernel<NANOVLLM_GEMM_B_KN>, grid, block, 0, s, a, b, c, p.m, p.n, p.k,
                            p.lda, p.ldb, p.ldc, int(tiles_n));
-    return check_launch("fp32_naive");
+    return check_launch("fp32_naive", 16, 16);
 }
 
 namespace {
 
 template <int BL, int BM, int BN, int BK, int MI, int CHN, int KW = 1>
-void launch_buffered(const Problem& p, hipStream_t s) {
+int launch_buffered(const Problem& p, hipStream_t s) {
     const int64_t tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
     hipLaunchKernelGGL((fp32_buffered_kernel<BL, BM, BN, BK, MI, CHN, KW>), dim3(static_cast<uint32_t>(tiles_m * tiles_n)),
                        dim3(256), 0, s, static_cast<const float*>(p.a), static_cast<const float*>(p.b),
                        static_cast<float*>(p.c), p.m, p.n, p.k, p.lda, p.ldb, p.ldc, int(tiles_m), int(tiles_n));
+    return check_launch("fp32_buffered", BM, BN);
 }
 
 template <int BL>
-void launch_buffered_for(const Problem& p, hipStream_t s) {
+int launch_buffered_for(const Problem& p, hipStream_t s) {
     const int64_t tiles64 = ((p.m + 63) / 64) * ((p.n + 63) / 64);
     const auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };   // on the busiest CU
     const auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
-    if (tiles(16, 32) <= 512) launch_buffered<BL, 16, 32, 64, 16, 1, 2>(p, s);
-    else if (tiles(32, 32) <= 512) launch_buffered<BL, 32, 32, 64, 16, 1, 2>(p, s);
-    else if (tiles64 < 512 && 2 * rounds(tiles64) <= rounds(tiles(32, 64))) {
-        if constexpr (BL == NANOVLLM_GEMM_B_KN) launch_buffered<BL, 64, 32, 64, 16, 1>(p, s);
-        else launch_buffered<BL, 64, 64, 32, 16, 1, 2>(p, s);
-    }
-    else if (tiles64 < 512) launch_buffered<BL, 32, 64, 32, 16, 1, 2>(p, s);
-    else launch_buffered<BL, 64, 64, 32, 32, 2>(p, s);
+    if (tiles(16, 32) <= 512) return launch_buffered<BL, 16, 32, 64, 16, 1, 2>(p, s);
+    if (tiles(32, 32) <= 512) return launch_buffered<BL, 32, 32, 64, 16, 1, 2>(p, s);
+    if (tiles64 >= 512) return launch_buffered<BL, 64, 64, 32, 32, 2>(p, s);
+    if (2 * rounds(tiles64) > rounds(tiles(32, 64))) return launch_buffered<BL, 32, 64, 32, 16, 1, 2>(p, s);
+    if constexpr (BL == NANOVLLM_GEMM_B_KN) return launch_buffered<BL, 64, 32, 64, 16, 1>(p, s);
+    else return launch_buffered<BL, 64, 64, 32, 16, 1, 2>(p, s);
 }
 
 }  // namespace
@@ -622,19 +621,15 @@ int launch_fp32_tiled(const Problem& p, hipStream_t s) {
     const bool buffered = aligned && ranges && (p.b_layout == NANOVLLM_GEMM_B_NK || p.n % 4 == 0);
     const int ti = int(tiles_m), tj = int(tiles_n);
     if (p.b_layout == NANOVLLM_GEMM_B_NK) {
-        if (buffered)
-            launch_buffered_for<NANOVLLM_GEMM_B_NK>(p, s);
-        else
-            hipLaunchKernelGGL(fp32_tiled_kernel<NANOVLLM_GEMM_B_NK>, grid, block, 0, s, a, b, c, p.m, p.n, p.k,
-                               p.lda, p.ldb, p.ldc, ti, tj);
+        if (buffered) return launch_buffered_for<NANOVLLM_GEMM_B_NK>(p, s);
+        hipLaunchKernelGGL(fp32_tiled_kernel<NANOVLLM_GEMM_B_NK>, grid, block, 0, s, a, b, c, p.m, p.n, p.k, p.lda,
+                           p.ldb, p.ldc, ti, tj);
     } else {
-        if (buffered)
-            launch_buffered_for<NANOVLLM_GEMM_B_KN>(p, s);
-        else
-            hipLaunchKernelGGL(fp32_tiled_kernel<NANOVLLM_GEMM_B_KN>, grid, block, 0, s, a, b, c, p.m, p.n, p.k,
-                               p.lda, p.ldb, p.ldc, ti, tj);
+        if (buffered) return launch_buffered_for<NANOVLLM_GEMM_B_KN>(p, s);
+        hipLaunchKernelGGL(fp32_tiled_kernel<NANOVLLM_GEMM_B_KN>, grid, block, 0, s, a, b, c, p.m, p.n, p.k, p.lda,
+                           p.ldb, p.ldc, ti, tj);
     }
-    return check_launch("fp32_tiled");
+    return check_launch("fp32_tiled", kT32BM, kT32BN);
 }
 
 }  // namespace nvg

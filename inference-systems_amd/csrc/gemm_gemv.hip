@@ -111,7 +111,7 @@ int launch_typed(const Problem& p, hipStream_t s) {
     if (per_lane <= 1) launch_unrolled<DT, DT_OUT, 1>(p, grid, s);
     else if (per_lane == 2) launch_unrolled<DT, DT_OUT, 2>(p, grid, s);
     else launch_unrolled<DT, DT_OUT, 4>(p, grid, s);
-    return check_launch("gemv_decode");
+    return check_launch("gemv_decode", 1, int(kGemvRows));
 }
 
 }  // namespace

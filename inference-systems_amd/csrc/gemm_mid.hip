@@ -93,7 +93,6 @@ __global__ __launch_bounds__(kThreads) void mfma_mid_kernel(
     }
     const int ktiles = static_cast<int>((k + kBK - 1) / kBK);
     const uint32_t lds0 = lds_address(ring);
-    using Yes = std::true_type;
     using No = std::false_type;
     // Copy j of K-tile t into `stage`; last_c: t may be the last K-tile.
     auto copy = [&](int t, int stage, int j, auto last_c) {
@@ -285,7 +284,7 @@ int launch_tile(const Problem& p, hipStream_t s) {
     hipLaunchKernelGGL((mfma_mid_kernel<DT, DT_OUT, EPI, RS, BN>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.m, p.n, p.k, p.lda,
                        p.ldb, p.c, p.ldc, c_vec, p.row_scale);
-    return check_launch("mfma_mid");
+    return check_launch("mfma_mid", kBM, BNO);
 }
 
 constexpr int64_t kCus = 256;

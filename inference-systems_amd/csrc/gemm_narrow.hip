@@ -17,8 +17,6 @@
 // 1024 x 3584 18.4 -> 13.9, gate/up pairs of 47 x (2 x 2624) x 1024 9.4 -> 6.3.
 #include "gemm_common.hpp"
 
-#include "gemm_common.hpp"
-
 namespace nvg {
 namespace {
 
@@ -245,7 +243,7 @@ int launch_tile(const Problem& p, hipStream_t s) {
                        dim3(static_cast<uint32_t>(tiles)), dim3(WGM * WGN * 64), 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.m, p.n, p.k, p.lda, p.ldb,
                        p.c, p.ldc, c_vec, p.row_scale);
-    return check_launch("mfma_narrow");
+    return check_launch("mfma_narrow", BM, BNO);
 }
 
 constexpr int64_t kCus = 256;

@@ -229,7 +229,7 @@ int launch_tile(const Problem& p, hipStream_t s) {
                        dim3(static_cast<uint32_t>(tiles_m * tiles_n)), dim3(WGM * WGN * 64), 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.c, p.m, p.n, p.k, p.lda,
                        p.ldb, p.ldc, int(tiles_m), int(tiles_n));
-    return check_launch("mfma_ragged");
+    return check_launch("mfma_ragged", BM, BN);
 }
 
 // Tiles by grid size.  A CU takes these unaligned loads at about 16 bytes per

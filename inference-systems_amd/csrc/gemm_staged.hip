@@ -564,7 +564,7 @@ int launch_tile(const Problem& p, hipStream_t s) {
     hipLaunchKernelGGL((mfma_staged_kernel<DT, DT_OUT, BM, BN, WGM, WGN, STAGES, EPI, RS, SP, KN>), grid, block, 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.m, p.n, p.k, p.lda,
                        p.ldb, p.c, p.ldc, c_vec, p.keys, p.row_scale, p.sample);
-    return check_launch("mfma_staged");
+    return check_launch("mfma_staged", BM, BNO);
 }
 
 // Tile and schedule by grid size (bf16, MI355X, one launch; every choice

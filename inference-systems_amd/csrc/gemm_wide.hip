@@ -327,7 +327,7 @@ int launch_tile(const Problem& p, hipStream_t s) {
     hipLaunchKernelGGL((mfma_wide_kernel<DT, DT_OUT, EPI, RS>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, s,
                        static_cast<const uint16_t*>(p.a), static_cast<const uint16_t*>(p.b), p.m, p.n, p.k, p.lda,
                        p.ldb, p.c, p.ldc, c_vec, p.row_scale);
-    return check_launch("mfma_wide");
+    return check_launch("mfma_wide", kBM, BNO);
 }
 
 template <int DT, int DT_OUT>

@@ -411,3 +411,20 @@ def test_add_rmsnorm_validates_before_launch(lib):
     rc = lib.nanovllm_gemm_add_rmsnorm_with_kernel(L.KERNEL_GEMV_DECODE, d, d, d, 1e-6, d, d, d, 40, 64, 512,
                                                    512, 512, 512, 64, 512, 0, BF16, BF16, None, 0, None)
     assert rc == L.EUNSUPPORTED and "gemv_decode" in L.last_error()
+
+
+def test_last_kernel_names_nothing_before_a_launch(lib):
+    """A refused call and a call without work launch nothing, so they leave the
+    thread's last kernel as it was (none, on a thread of its own)."""
+    import threading
+    seen = []
+
+    def calls():
+        seen.append(L.last_kernel())
+        lib.nanovllm_gemm(None, None, None, 0, 8, 8, 8, 8, 8, NK, BF16, BF16, None)
+        lib.nanovllm_gemm(None, None, None, 8, 8, 0, 8, 8, 8, NK, BF16, BF16, None)
+        seen.append(L.last_kernel())
+    t = threading.Thread(target=calls)
+    t.start()
+    t.join()
+    assert seen == ["", ""]

@@ -1,0 +1,43 @@
+"""GPU tests of which kernel and tile a problem runs on: shapes on both sides of
+the dispatch rules (nanovllm_gemm_last_kernel names what the call launched).
+Every form of a kernel id gives the same bits, so only the names, and the time,
+tell a wrong rule."""
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+from conftest import PKG
+from test_gemm_gpu import DEV, _say
+
+pytestmark = pytest.mark.gpu
+
+L = PKG._lib
+G = importlib.import_module("inference_systems_amd.kernels.gemm")
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def ran(m, n, k, dtype=BF16, out=None, kn=False, silu=False):
+    a = torch.zeros((m, k), dtype=dtype, device=DEV)
+    w = torch.zeros((k, n) if kn else (2 * n if silu else n, k), dtype=dtype, device=DEV)
+    _say(f"last kernel {m}x{n}x{k} kn={kn} silu={silu}")
+    if silu:
+        G.gemm_silu_mul(a, w, out)
+    else:
+        (G.gemm_kn if kn else G.gemm)(a, w, out)
+    torch.cuda.synchronize()
+    return L.last_kernel()
+
+
+@pytest.mark.parametrize("m,n,k,dtype,want", [
+    (1, 512, 256, BF16, "gemv_decode 1x"), (4, 512, 256, BF16, "splitk_decode 8x16"),
+    (32, 8192, 256, BF16, "splitk_decode 32x32"), (200, 1024, 512, BF16, "mfma_narrow 32x32"),
+    (2048, 4096, 1024, BF16, "mfma_mid 128x256"), (4096, 1024, 1024, F16, "mfma_mid 128x128"),
+    (4096, 4096, 512, BF16, "mfma_wide 256x256"), (2048, 4096, 128, BF16, "mfma_staged 128x256"),
+    (100, 100, 101, BF16, "mfma_ragged 32x32"), (5, 5, 5, BF16, "mfma_direct 64x64"),
+    (100, 128, 128, F32, "fp32_buffered 16x32"), (100, 128, 127, F32, "fp32_tiled 64x64"),
+])
+def test_kernel_families(m, n, k, dtype, want):
+    assert ran(m, n, k, dtype).startswith(want)
