@@ -1,6 +1,6 @@
-// mfma_narrow: mfma_staged's form for grids of at most one round on the CUs,
-// C[M,N] = A[M,K] * W[N,K]^T (or B[K,N]) on tiles down to 32 x 32.  Such a
-// grid is bound by the chain of K-tiles in each workgroup (copies, barrier,
+// mfma_narrow: mfma_staged's form for grids of at most one round on the CUs, from a
+// K that grows with the tile, C[M,N] = A[M,K] * W[N,K]^T (or B[K,N]) on tiles
+// down to 32 x 32.  Such a grid is bound by the chain of K-tiles in each workgroup (copies, barrier,
 // fragment reads, MFMAs; 0.27 us per 64 elements of K on 4 waves of 64 x 64,
 // however deep the ring), so:
 //   * tiles are as small as fills the CUs once: fewer bytes copied and read
@@ -288,6 +288,33 @@ int launch_silu(const Problem& p, hipStream_t s) {
     return launch_tile<DT, DT_OUT, 64, 64, 1, 2, 2, 4, EPI_SILU_MUL, RS, 0>(p, s);
 }
 
+// Which plain grids take these tiles, up to one round of 64 x 64.  A long
+// K-tile fills and drains once per workgroup, so they need a K to spread that
+// over; more of it where 8 waves share the tile, and where rows of A and B are
+// not whole 128-byte lines, which adds a line to most copy instructions of
+// every K-tile (mfma_staged's 64 x 64 against these, bf16 and f16, us):
+//   * 32 x 32: 983 x 256 x 64 3.25 / 3.41, 795 x 128 x 96 3.43 / 3.29;
+//   * 32 x 64: K = 320 544 x 832 4.15 / 4.32, 384 573 x 832 4.60 / 4.32, 512
+//     312 x 1600 5.00 / 4.70; rows of other lengths: K = 552 2259 x 192 5.00 /
+//     5.44, 584 245 x 1472 5.67 / 5.31, 608 517 x 576 5.48 / 5.17;
+//   * 64 x 64: K = 448 264 x 2816 5.01 / 5.34, 512 67 x 5248 5.27 / 4.89, 1024 842
+//     x 704 7.34 / 6.64; rows of other lengths: K = 816 395 x 2240 6.64 / 7.22, 1456
+//     452 x 1856 9.25 / 9.82, 1848 1727 x 448 11.84 / 11.66, 2016 203 x 3264 11.56 /
+//     10.88;
+//   * B[K,N], 32 x 64: K = 320 78 x 832 4.12 / 4.31, 512 447 x 192 4.80 / 4.56;
+//     rows of other lengths: K = 560 83 x 3912 5.95 / 6.23, 768 149 x 592 6.32 /
+//     5.82; 64 x 64: K = 704 2619 x 384 6.30 / 6.60, 1024 1272 x 512 7.40 / 7.13,
+//     1152 237 x 2112 7.83 / 7.20; rows of other lengths: K = 1160 132 x 3696 8.84
+//     / 9.43, 2256 56 x 11520 18.0 / 17.1.
+bool plain_pays(const Problem& p) {
+    if (tiles(p, 64, 64) > kCus) return false;
+    const bool lines = p.lda % 64 == 0 && p.ldb % 64 == 0;
+    const bool rows32 = tiles(p, 32, 64) <= kCus;
+    if (p.b_layout == NANOVLLM_GEMM_B_KN) return p.k >= (rows32 ? (lines ? 512 : 768) : (lines ? 1024 : 2048));
+    if (tiles(p, 32, 32) <= kCus) return p.k > 64;
+    return p.k >= (rows32 ? (lines ? 384 : 576) : (lines ? 512 : 1792));
+}
+
 template <int DT, int DT_OUT>
 int launch_typed(const Problem& p, hipStream_t s) {
     if (p.b_layout == NANOVLLM_GEMM_B_KN) return launch_plain<DT, DT_OUT, EPI_NONE, 0, 1>(p, s);
@@ -301,13 +328,12 @@ int launch_typed(const Problem& p, hipStream_t s) {
 
 }  // namespace
 
-// The grids of launch_plain's and launch_silu's largest tiles.  K-tiles are
-// counted in 32 bits.
+// K-tiles are counted in 32 bits.
 bool mfma_narrow_pays(const Problem& p) {
     if (p.k >= (int64_t(1) << 30)) return false;
     if (p.b_layout == NANOVLLM_GEMM_B_KN && (p.epi != EPI_NONE || p.row_scale != nullptr)) return false;
     if (p.epi == EPI_SILU_MUL) return tiles(p, 64, 32) <= 2 * kCus;
-    return p.epi == EPI_NONE && tiles(p, 64, 64) <= kCus;
+    return p.epi == EPI_NONE && plain_pays(p);
 }
 
 int launch_mfma_narrow(const Problem& p, hipStream_t s) {

@@ -571,8 +571,9 @@ int launch_tile(const Problem& p, hipStream_t s) {
 // sums K in the same order, so none changes a result bit).  "tiles" counts
 // 128 x 128 tiles, "wide" 128 x 256 ones:
 //   * grids of at most one round of 64 x 64 tiles (SiLU pairs: two of 64 x
-//     32 outputs): the smaller tiles of gemm_narrow.hip, by the rules there;
-//   * tiles <= 128 (half the CUs) above that: 64 x 64 tiles, four times the
+//     32 outputs) from a K that grows with the tile: the smaller tiles of
+//     gemm_narrow.hip, by the rules there;
+//   * tiles <= 128 (half the CUs) otherwise: 64 x 64 tiles, four times the
 //     workgroups (512 x 4096 x 1024 12.3 -> 8.1 us, 2048 x 1024 x 2048 20.6 ->
 //     13.8 us), on a 3-deep ring with spread copies (against a 2-deep burst
 //     ring: 512 x 4096 x 1024 8.49 -> 8.04, 256 x 6144 x 1024 8.03 -> 7.46,

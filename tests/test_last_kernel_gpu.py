@@ -41,3 +41,25 @@ def ran(m, n, k, dtype=BF16, out=None, kn=False, silu=False):
 ])
 def test_kernel_families(m, n, k, dtype, want):
     assert ran(m, n, k, dtype).startswith(want)
+
+
+@pytest.mark.parametrize("m,n,k,kn,want", [
+    # one round of 32 x 32 tiles
+    (128, 512, 64, False, "mfma_staged 64x64"), (128, 512, 72, False, "mfma_narrow 32x32"),
+    # of 32 x 64: rows of whole 128-byte lines, then not
+    (320, 1536, 320, False, "mfma_staged 64x64"), (320, 1536, 384, False, "mfma_narrow 32x64"),
+    (320, 1536, 568, False, "mfma_staged 64x64"), (320, 1536, 584, False, "mfma_narrow 32x64"),
+    # of 64 x 64
+    (700, 1024, 448, False, "mfma_staged 64x64"), (700, 1024, 512, False, "mfma_narrow 64x64"),
+    (700, 1024, 1784, False, "mfma_staged 64x64"), (700, 1024, 1800, False, "mfma_narrow 64x64"),
+    # more than one round
+    (1024, 2048, 512, False, "mfma_staged 64x64"),
+    # B[K,N]
+    (200, 512, 448, True, "mfma_staged 64x64"), (200, 512, 512, True, "mfma_narrow 32x64"),
+    (200, 520, 760, True, "mfma_staged 64x64"), (200, 520, 768, True, "mfma_narrow 32x64"),
+    (700, 1024, 960, True, "mfma_staged 64x64"), (700, 1024, 1024, True, "mfma_narrow 64x64"),
+    (700, 1000, 2040, True, "mfma_staged 64x64"), (700, 1000, 2048, True, "mfma_narrow 64x64"),
+])
+def test_small_grids(m, n, k, kn, want):
+    """A short K stays on the 64 x 64 tiles with 64-element K-tiles."""
+    assert ran(m, n, k, kn=kn) == want

@@ -27,15 +27,28 @@ NK = [(1, 8, 8, 9000), (33, 100, 120, 4400), (31, 1000, 136, 4400), (40, 96, 100
       (190, 4100, 72, 1500)]
 KN = [(33, 104, 120, 4400), (90, 4104, 136, 1100), (321, 1000, 648, 4400), (190, 4104, 72, 1500)]
 
+# The shapes above whose K is too short for a tile of that size run
+# mfma_staged's; these run the tiles they name (K of whole K-tiles of 128, and
+# with tails of one chunk, of half a K-tile and more).
+FORMS = [("NK", 40, 96, 72, 4400, "32x32"), ("NK", 65, 333, 1800, 4400, "32x32"),
+         ("NK", 90, 4104, 584, 1100, "32x64"), ("NK", 321, 1001, 648, 4400, "32x64"),
+         ("NK", 320, 1472, 384, 4400, "32x64"), ("NK", 500, 1029, 1800, 4400, "64x64"),
+         ("NK", 190, 4100, 512, 1500, "64x64"), ("NK", 449, 1500, 576, 3000, "64x64"),
+         ("KN", 33, 104, 776, 4400, "32x64"), ("KN", 90, 4104, 840, 1100, "32x64"), ("KN", 200, 512, 512, 4400, "32x64"),
+         ("KN", 190, 4104, 2056, 1500, "64x64"), ("KN", 449, 1472, 1088, 3000, "64x64")]
 
-def _run(m, n, k, mm, din, dout, layout):
+
+def _run(m, n, k, mm, din, dout, layout, tile=None):
     gen = torch.Generator().manual_seed(m + n + k)
     a = torch.randn((mm, k), generator=gen).to(din)
     b = (torch.randn((n, k) if layout == L.B_NK else (k, n), generator=gen) * 0.1).to(din)
     ad, bd = a.to(DEV), b.to(DEV)
     _say(f"narrow M={m} N={n} K={k} layout={layout} {NAME[din]}->{NAME[dout]}")
     out = G.gemm_with_kernel(ad[:m], bd, L.KERNEL_MFMA_STAGED, dout, layout)
+    if tile is not None:
+        assert L.last_kernel() == f"mfma_narrow {tile}"
     big = G.gemm_with_kernel(ad, bd, L.KERNEL_MFMA_STAGED, dout, layout)
+    assert tile is None or not L.last_kernel().startswith("mfma_narrow")
     torch.cuda.synchronize()
     assert torch.equal(out, big[:m]), f"{int((out != big[:m]).sum())} outputs differ"
     _check_tolerance(out.cpu(), a[:m], b, layout, dout)
@@ -51,6 +64,12 @@ def test_narrow_nk(m, n, k, mm, din, dout):
 @pytest.mark.parametrize("din,dout", [(BF16, BF16), (F16, F32)], ids=["bf16", "f16-f32"])
 def test_narrow_kn(m, n, k, mm, din, dout):
     _run(m, n, k, mm, din, dout, L.B_KN)
+
+
+@pytest.mark.parametrize("layout,m,n,k,mm,tile", FORMS, ids=lambda v: str(v))
+@pytest.mark.parametrize("din,dout", [(BF16, BF16), (F16, F32)], ids=["bf16", "f16-f32"])
+def test_narrow_forms(layout, m, n, k, mm, tile, din, dout):
+    _run(m, n, k, mm, din, dout, L.B_NK if layout == "NK" else L.B_KN, tile)
 
 
 # Rows x outputs: 32 x 32, 64 x 32 on 8 waves, 64 x 32 two to a CU.
