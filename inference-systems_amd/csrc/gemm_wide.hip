@@ -355,7 +355,10 @@ int launch_typed(const Problem& p, hipStream_t s) {
 // of 128 x 256 28.6 / 25.3, 320 28.5 / 25.7, 416 31.5 / 28.9, 896 (SiLU pairs) 66.0 /
 // 59.4, 1579 x 4992 (260, and 507 of 128 x 128) 21.6 / 24.6 (not taken), 576 44.4 /
 // 50.2 and 768 49.4 / 53.5 (not taken); K = 512: 416 20.4 / 19.2, 768 31.9 / 34.3
-// (not taken); K = 3072: 272 68.2 / 59.7, 576 109 / 123 (not taken).
+// (not taken); K = 3072: 272 68.2 / 59.7, 576 109 / 123 (not taken).  Up to 8
+// K-tiles the model has to promise 7%: a partial round there costs more than it
+// says (K = 256: 624 tiles of 128 x 256 (f16) 21.1 / 23.1, 750 21.6 / 23.8, 646 (SiLU
+// pairs) 25.4 / 26.3; K = 480, 1050 (f16) 59.9 / 61.3; not taken).
 bool mfma_wide_pays(const Problem& p) {
     if (p.b_layout != NANOVLLM_GEMM_B_NK || p.k < 256 || p.k > (int64_t(1) << 30)) return false;
     if (p.epi != EPI_NONE && p.epi != EPI_SILU_MUL) return false;
@@ -378,7 +381,7 @@ bool mfma_wide_pays(const Problem& p) {
     int64_t narrow_cost =
         160 + narrow / kCus * (480 + 73 * kt) + (part > 0 ? 220 + 48 * kt + part * (120 + 27 * kt) / kCus : 0);
     if (tiles128 <= 2 * kCus && 400 + 108 * kt < narrow_cost) narrow_cost = 400 + 108 * kt;
-    return wide_cost < narrow_cost;
+    return wide_cost * 100 < narrow_cost * (kt <= 8 ? 93 : 100);
 }
 
 int launch_mfma_wide(const Problem& p, hipStream_t s) {

@@ -63,3 +63,14 @@ def test_kernel_families(m, n, k, dtype, want):
 def test_small_grids(m, n, k, kn, want):
     """A short K stays on the 64 x 64 tiles with 64-element K-tiles."""
     assert ran(m, n, k, kn=kn) == want
+
+
+@pytest.mark.parametrize("m,n,k,silu,want", [
+    # one part of a round, and one full round and a part: by the model's margin at a short K
+    (4096, 2560, 256, False, "mfma_wide 256x256"), (6300, 3648, 256, False, "mfma_mid 128x256"),
+    (4757, 2112, 256, True, "mfma_mid 128x128"), (3010, 2688, 320, True, "mfma_wide 256x128"),
+    (5321, 6312, 480, False, "mfma_mid 128x256"),
+    (5321, 6312, 1024, False, "mfma_wide 256x256"),
+])
+def test_large_grids(m, n, k, silu, want):
+    assert ran(m, n, k, silu=silu) == want
