@@ -315,6 +315,19 @@ bool plain_pays(const Problem& p) {
     return p.k >= (rows32 ? (lines ? 384 : 576) : (lines ? 512 : 1792));
 }
 
+// SiLU pairs: all grids of one round of 64 x 32 outputs; up to two rounds, where
+// a workgroup of 64 x 32 copies as many rows of A as W rows, mfma_staged's 64 x 64
+// outputs copy less and win where rows are not whole 128-byte lines (unless only
+// its 128 x 128 tiles are left) and on a very long K (these / those, bf16, us:
+// 729 x 1216 x 992 10.7 / 10.3, norm + 827 x 1024 x 616 12.7 / 11.9, norm + 59 x 9344
+// x 3968 45.5 / 43.8; taken: 929 x 736 x 1024 9.1 / 10.0).
+bool silu_pays(const Problem& p) {
+    if (tiles(p, 64, 32) <= kCus) return true;
+    if (tiles(p, 64, 32) > 2 * kCus || p.k > 3072) return false;
+    const int64_t tiles128 = (p.m + 127) / 128 * ((2 * p.n + 127) / 128);
+    return (p.lda % 64 == 0 && p.ldb % 64 == 0) || tiles128 > kCus / 2;
+}
+
 template <int DT, int DT_OUT>
 int launch_typed(const Problem& p, hipStream_t s) {
     if (p.b_layout == NANOVLLM_GEMM_B_KN) return launch_plain<DT, DT_OUT, EPI_NONE, 0, 1>(p, s);
@@ -332,7 +345,7 @@ int launch_typed(const Problem& p, hipStream_t s) {
 bool mfma_narrow_pays(const Problem& p) {
     if (p.k >= (int64_t(1) << 30)) return false;
     if (p.b_layout == NANOVLLM_GEMM_B_KN && (p.epi != EPI_NONE || p.row_scale != nullptr)) return false;
-    if (p.epi == EPI_SILU_MUL) return tiles(p, 64, 32) <= 2 * kCus;
+    if (p.epi == EPI_SILU_MUL) return silu_pays(p);
     return p.epi == EPI_NONE && plain_pays(p);
 }
 

@@ -577,7 +577,8 @@ int launch_tile(const Problem& p, hipStream_t s) {
 //     workgroups (512 x 4096 x 1024 12.3 -> 8.1 us, 2048 x 1024 x 2048 20.6 ->
 //     13.8 us), on a 3-deep ring with spread copies (against a 2-deep burst
 //     ring: 512 x 4096 x 1024 8.49 -> 8.04, 256 x 6144 x 1024 8.03 -> 7.46,
-//     2048 x 1024 x 2048 14.2 -> 14.0);
+//     2048 x 1024 x 2048 14.2 -> 14.0); SiLU pairs, which need two 32-row W blocks
+//     per wave, 64 x 64 outputs on 64 x 128 tiles of the same schedule;
 //   * 128 < wide <= 256 or wide > 384: one 8-wave workgroup per CU on
 //     128 x 256 (half the A reads of two 128 x 128 tiles), 3-deep ring,
 //     copies spread between the MFMAs.  Against the 2-deep 128 x 128 burst
@@ -609,6 +610,8 @@ int launch_epi(const Problem& p, hipStream_t s) {
     const int64_t tiles = ((p.m + 127) / 128) * ((n_tiles + 127) / 128);
     if constexpr (EPI == EPI_NONE)
         if (tiles <= kSmallGridTiles) return launch_tile<DT, DT_OUT, 64, 64, 2, 2, 3, EPI, RS, 1>(p, s);
+    if constexpr (EPI == EPI_SILU_MUL)
+        if (tiles <= kSmallGridTiles) return launch_tile<DT, DT_OUT, 64, 128, 2, 2, 3, EPI, RS, 1>(p, s);
     const int64_t wide = ((p.m + 127) / 128) * ((n_tiles + 255) / 256);
     const bool head_loses = EPI == EPI_ARGMAX && p.sample.temperature != nullptr && wide > kCus && p.m <= 128;
     if (wide > kCus / 2 && (wide <= kCus || wide > 3 * kCus / 2) && !head_loses)

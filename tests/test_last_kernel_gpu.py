@@ -74,3 +74,24 @@ def test_small_grids(m, n, k, kn, want):
 ])
 def test_large_grids(m, n, k, silu, want):
     assert ran(m, n, k, silu=silu) == want
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (200, 1200, 264, "mfma_narrow 64x32"), (100, 1000, 264, "mfma_narrow 32x32"),
+    # two rounds of 64 x 32 outputs: whole 128-byte lines, not, a very long K, and
+    # more than 128 tiles of 128 x 128
+    (729, 1216, 1024, "mfma_narrow 64x32"), (729, 1216, 992, "mfma_staged 64x64"),
+    (200, 3584, 3072, "mfma_narrow 64x32"), (200, 3584, 3136, "mfma_staged 64x64"),
+    (440, 2080, 992, "mfma_narrow 64x32"),
+])
+def test_small_silu_grids(m, n, k, want):
+    assert ran(m, n, k, silu=True) == want
+
+
+@pytest.mark.parametrize("m,n,k,kn,want", [
+    (100, 100, 15, False, "mfma_direct 64x64"), (100, 100, 17, False, "mfma_ragged 32x32"),
+    (1500, 1001, 23, True, "mfma_direct 64x64"), (1500, 1001, 25, True, "mfma_ragged 32x64"),
+    (1500, 1001, 25, False, "mfma_ragged 32x64"), (100, 7, 65, True, "mfma_direct 64x64"),
+])
+def test_ragged_grids(m, n, k, kn, want):
+    assert ran(m, n, k, kn=kn) == want

@@ -72,11 +72,13 @@ def test_narrow_forms(layout, m, n, k, mm, tile, din, dout):
     _run(m, n, k, mm, din, dout, L.B_NK if layout == "NK" else L.B_KN, tile)
 
 
-# Rows x outputs: 32 x 32, 64 x 32 on 8 waves, 64 x 32 two to a CU.
-@pytest.mark.parametrize("m,n,k", [(40, 1000, 136), (33, 8, 520), (70, 3000, 72), (200, 3333, 264)],
-                         ids=lambda v: str(v))
+# Rows x outputs: 32 x 32, 64 x 32 on 8 waves, 64 x 32 two to a CU, and
+# mfma_staged's 64 x 64 where rows of that grid are not whole 128-byte lines.
+@pytest.mark.parametrize("m,n,k,tile", [
+    (40, 1000, 136, "narrow 32x32"), (33, 8, 520, "narrow 32x32"), (70, 3000, 72, "narrow 64x32"),
+    (200, 3333, 320, "narrow 64x32"), (200, 3333, 264, "staged 64x64")], ids=lambda v: str(v))
 @pytest.mark.parametrize("norm", [False, True], ids=["plain", "add-norm"])
-def test_narrow_silu(m, n, k, norm):
+def test_narrow_silu(m, n, k, tile, norm):
     mm = 3000
     gen = torch.Generator().manual_seed(m + n + k)
     a = torch.randn((mm, k), generator=gen).bfloat16()
@@ -88,7 +90,9 @@ def test_narrow_silu(m, n, k, norm):
         run = lambda x: K.gemm_add_rmsnorm_with_kernel(x, x, nw, wd, 1e-6, L.KERNEL_MFMA_STAGED, silu_mul=True)[0]  # noqa: E731
     else:
         run = lambda x: G.gemm_silu_mul_with_kernel(x, wd, L.KERNEL_MFMA_STAGED)  # noqa: E731
-    out, big = run(ad[:m]), run(ad)
+    out = run(ad[:m])
+    assert L.last_kernel() == f"mfma_{tile}"
+    big = run(ad)
     torch.cuda.synchronize()
     assert torch.equal(out, big[:m]), f"{int((out != big[:m]).sum())} outputs differ"
     if not norm:
