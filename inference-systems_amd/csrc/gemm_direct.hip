@@ -6,9 +6,9 @@
 // partial tiles (gemm_bench.cu:92), K that is not a multiple of 16, odd
 // strides and unaligned pointers.  It is the selection table's fallback for
 // any half-precision problem the faster kernels cannot take: those run
-// gemm_ragged.hip's tiles, and only rows shorter than one 16-byte chunk (K or,
-// on B[K,N], N below 8) the kernel here, which also runs any problem asked of
-// it by name.
+// gemm_ragged.hip's tiles, and only a K of a few elements (and, on B[K,N], rows
+// of less than one 16-byte chunk) the kernel here, which also runs any problem
+// of whole chunks asked of it by name.
 #include "gemm_common.hpp"
 
 namespace nvg {

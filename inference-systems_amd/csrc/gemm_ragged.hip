@@ -263,9 +263,14 @@ int launch_typed(const Problem& p, hipStream_t s) {
 
 }  // namespace
 
-// One whole chunk per row of every operand, and K-tiles counted in 32 bits.
+// One whole chunk per row of every operand, and K-tiles counted in 32 bits.  On a
+// K of a few elements a K-tile is mostly zeros, and mfma_direct's element loads are
+// fewer (mfma_direct / these, bf16 and f16, us: 1482 x 925 x 11 (B[K,N]) 4.9 / 6.6,
+// 469 x 841 x 15 4.0 / 4.5, 458 x 89 x 17 4.4 / 3.9; large grids 2499 x 1731 x 23
+// (B[K,N]) 9.0 / 10.2, 415 x 6060 x 51 14.0 / 7.3).
 bool mfma_ragged_ok(const Problem& p) {
-    return p.k >= 8 && p.k < (int64_t(1) << 30) && (p.b_layout == NANOVLLM_GEMM_B_NK || p.n >= 8);
+    const int64_t tiles32 = (p.m + 31) / 32 * ((p.n + 31) / 32);
+    return p.k > (tiles32 <= 512 ? 16 : 24) && p.k < (int64_t(1) << 30) && (p.b_layout == NANOVLLM_GEMM_B_NK || p.n >= 8);
 }
 
 int launch_mfma_ragged(const Problem& p, hipStream_t s) {

@@ -27,11 +27,12 @@ def _framed(x, pad, offset):
     return buf, buf.data_ptr() + offset * x.element_size(), ld
 
 
-# Tiles: 32 x 32 (small grids), 16 x 32 (M <= 16, 260 tiles of it), 32 x 64
-# (514 tiles of 32 x 32) and 64 x 64 (513 of 64 x 64); K of one chunk, one
-# element more, and around the ends of 64- and 128-element K-tiles and of the
-# K-tiles loaded ahead (up to four).
-SHAPES = [(1, 8, 8), (33, 31, 9), (31, 33, 15), (5, 70, 63), (32, 32, 65), (40, 100, 127), (64, 65, 129),
+# Tiles: 32 x 32 (small grids), 16 x 32 (M <= 16, 261 tiles of it), 32 x 64
+# (514 tiles of 32 x 32) and 64 x 64 (528 of 64 x 64); K of two chunks and one
+# element more, less than three, and around the ends of 64- and 128-element
+# K-tiles and of the K-tiles loaded ahead (up to four); up to 16 elements run
+# mfma_direct's own kernel.
+SHAPES = [(1, 8, 8), (33, 31, 9), (31, 33, 15), (33, 31, 17), (31, 33, 23), (47, 130, 31), (5, 70, 63), (32, 32, 65), (40, 100, 127), (64, 65, 129),
           (70, 33, 257), (17, 50, 391), (3, 9, 520), (16, 8321, 131), (63, 8209, 72 + 1), (1000, 2051, 67)]
 
 
