@@ -267,10 +267,23 @@ int launch_typed(const Problem& p, hipStream_t s) {
 // K of a few elements a K-tile is mostly zeros, and mfma_direct's element loads are
 // fewer (mfma_direct / these, bf16 and f16, us: 1482 x 925 x 11 (B[K,N]) 4.9 / 6.6,
 // 469 x 841 x 15 4.0 / 4.5, 458 x 89 x 17 4.4 / 3.9; large grids 2499 x 1731 x 23
-// (B[K,N]) 9.0 / 10.2, 415 x 6060 x 51 14.0 / 7.3).
+// (B[K,N]) 9.0 / 10.2, 2836 x 704 x 31 7.0 / 7.6, 4466 x 1677 x 33 21.6 / 12.6).
+// B[K,N] behind rows of A that are aligned chunks needs more: mfma_direct reads
+// those 16 bytes at a time, and its 64 x 64 tiles read B less often than 32 x 64,
+// which tells while their last round is fuller than half: 284 x 5482 x 64 4.9 /
+// 7.2, 7 x 4715 x 64 3.2 / 3.5, 16 x 7001 x 96 4.5 / 3.7; 646 x 2485 x 192 (429 tiles
+// of 64 x 64) 8.3 / 10.1, 7672 x 119 x 256 (240) 6.7 / 7.3, 745 x 1861 x 128 (360) 6.5 /
+// 5.8, 2854 x 470 x 256 9.4 / 7.3; 967 x 6951 x 72 11.2 / 14.5, 1313 x 2671 x 128 11.2
+// / 8.4.
 bool mfma_ragged_ok(const Problem& p) {
-    const int64_t tiles32 = (p.m + 31) / 32 * ((p.n + 31) / 32);
-    return p.k > (tiles32 <= 512 ? 16 : 24) && p.k < (int64_t(1) << 30) && (p.b_layout == NANOVLLM_GEMM_B_NK || p.n >= 8);
+    const auto tiles = [&](int64_t t) { return (p.m + t - 1) / t * ((p.n + t - 1) / t); };
+    const bool a_chunks = reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && p.lda % 8 == 0 && p.k % 8 == 0;
+    int64_t least = tiles(32) <= 512 ? 17 : 33;   // K
+    if (p.b_layout == NANOVLLM_GEMM_B_KN && a_chunks) {
+        const int64_t t64 = tiles(64);
+        least = tiles(32) <= 512 ? 65 : t64 > 512 ? 88 : t64 <= 256 || t64 > 384 ? 257 : 65;
+    }
+    return p.k >= least && p.k < (int64_t(1) << 30) && (p.b_layout == NANOVLLM_GEMM_B_NK || p.n >= 8);
 }
 
 int launch_mfma_ragged(const Problem& p, hipStream_t s) {

@@ -90,8 +90,14 @@ def test_small_silu_grids(m, n, k, want):
 
 @pytest.mark.parametrize("m,n,k,kn,want", [
     (100, 100, 15, False, "mfma_direct 64x64"), (100, 100, 17, False, "mfma_ragged 32x32"),
-    (1500, 1001, 23, True, "mfma_direct 64x64"), (1500, 1001, 25, True, "mfma_ragged 32x64"),
-    (1500, 1001, 25, False, "mfma_ragged 32x64"), (100, 7, 65, True, "mfma_direct 64x64"),
+    (1500, 1001, 31, True, "mfma_direct 64x64"), (1500, 1001, 33, True, "mfma_ragged 32x64"),
+    (1500, 1001, 33, False, "mfma_ragged 32x64"), (100, 7, 65, True, "mfma_direct 64x64"),
+    # B[K,N] behind rows of A that are aligned chunks: 35, 340, 400 and 768 tiles
+    # of 64 x 64
+    (300, 401, 64, True, "mfma_direct 64x64"), (300, 401, 72, True, "mfma_ragged 32x32"),
+    (1270, 1051, 64, True, "mfma_direct 64x64"), (1270, 1051, 72, True, "mfma_ragged 32x64"),
+    (1270, 1251, 256, True, "mfma_direct 64x64"), (1270, 1251, 264, True, "mfma_ragged 32x64"),
+    (2048, 1501, 80, True, "mfma_direct 64x64"), (2048, 1501, 88, True, "mfma_ragged 64x64"),
 ])
 def test_ragged_grids(m, n, k, kn, want):
     assert ran(m, n, k, kn=kn) == want
