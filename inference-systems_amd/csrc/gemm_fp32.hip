@@ -17,6 +17,8 @@
 //                 into a double-buffered LDS tile).
 #include <type_traits>
 
+#include <algorithm>
+
 #include "gemm_common.hpp"
 
 namespace nvg {
@@ -244,7 +246,13 @@ __global__ __launch_bounds__(kT32Threads) void fp32_tiled_kernel(
 //     4096 x 1024 29.5 -> 26.3 (33.0), 1400 x 1300 x 512 (924 / 462) 22.2 -> 20.4
 //     (32 x 64 23.9), 1024^3 21.0 -> 20.2.  B[K,N] reads its fragments a float
 //     at a time, so there 64 x 32 with one chain stays instead of 64 x 64 (1024^3
-//     19.7 against 20.1, 222 x 3648 x 960 20.4 / 20.8);
+//     19.7 against 20.1, 222 x 3648 x 960 20.4 / 20.8), as it does below K = 200 (346
+//     x 2436 x 40 4.9 / 5.7, 186 x 5148 x 92 6.1 / 6.5);
+//   * 64 x 32 where that puts less on the busiest CU than either (B[K,N] 1816 x
+//     524 x 2728, 493 workgroups, 513 of 32 x 64: 46.2 / 65.8), and instead of 32 x
+//     32 where those fit one round and B is larger than the L2s, so that reading
+//     it for half as many rows at a time costs (56 x 5316 x 6928 59.4 / 67.3, 167 x
+//     1892 x 7208 60.4 / 64.8; not below: 2286 x 172 x 5680 50.1 / 46.7);
 //   * from 512 tiles of 64 x 64: those, v_mfma_f32_32x32x2_f32 in two accumulator
 //     chains (odd steps in the second, added before the store), BK = 32 (2048^3
 //     156.7 -> 126.6 us, 4096^3 1208.6 -> 966.6 us).
@@ -587,17 +595,25 @@ int launch_buffered(const Problem& p, hipStream_t s) {
     return check_launch("fp32_buffered", BM, BN);
 }
 
+constexpr int64_t kL2Bytes = int64_t(32) << 20;   // of the 8 XCDs together
+
 template <int BL>
 int launch_buffered_for(const Problem& p, hipStream_t s) {
     const int64_t tiles64 = ((p.m + 63) / 64) * ((p.n + 63) / 64);
     const auto rounds = [](int64_t workgroups) { return (workgroups + 255) / 256; };   // on the busiest CU
     const auto tiles = [&](int64_t bm, int64_t bn) { return ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn); };
     if (tiles(16, 32) <= 512) return launch_buffered<BL, 16, 32, 64, 16, 1, 2>(p, s);
-    if (tiles(32, 32) <= 512) return launch_buffered<BL, 32, 32, 64, 16, 1, 2>(p, s);
+    if (tiles(32, 32) <= 512) {
+        if (tiles(64, 32) <= 256 && p.n * p.k * 4 > kL2Bytes) return launch_buffered<BL, 64, 32, 64, 16, 1, 2>(p, s);
+        return launch_buffered<BL, 32, 32, 64, 16, 1, 2>(p, s);
+    }
     if (tiles64 >= 512) return launch_buffered<BL, 64, 64, 32, 32, 2>(p, s);
-    if (2 * rounds(tiles64) > rounds(tiles(32, 64))) return launch_buffered<BL, 32, 64, 32, 16, 1, 2>(p, s);
-    if constexpr (BL == NANOVLLM_GEMM_B_KN) return launch_buffered<BL, 64, 32, 64, 16, 1>(p, s);
-    else return launch_buffered<BL, 64, 64, 32, 16, 1, 2>(p, s);
+    const int64_t r64 = 2 * rounds(tiles64), r32 = rounds(tiles(32, 64));
+    if (rounds(tiles(64, 32)) < std::min(r64, r32)) return launch_buffered<BL, 64, 32, 64, 16, 1, 2>(p, s);
+    if (r64 > r32) return launch_buffered<BL, 32, 64, 32, 16, 1, 2>(p, s);
+    if constexpr (BL == NANOVLLM_GEMM_B_NK)
+        if (p.k >= 200) return launch_buffered<BL, 64, 64, 32, 16, 1, 2>(p, s);
+    return launch_buffered<BL, 64, 32, 64, 16, 1>(p, s);
 }
 
 }  // namespace

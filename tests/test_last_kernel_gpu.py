@@ -101,3 +101,16 @@ def test_small_silu_grids(m, n, k, want):
 ])
 def test_ragged_grids(m, n, k, kn, want):
     assert ran(m, n, k, kn=kn) == want
+
+
+@pytest.mark.parametrize("m,n,k,kn,want", [
+    (16, 4096, 256, False, "16x32"), (200, 2044, 260, False, "32x32"), (200, 2044, 260, True, "32x32"),
+    # B of more and of less than 32 MiB, in one round of 64 x 32 tiles or more
+    (56, 5316, 1580, False, "64x32"), (56, 5316, 1576, False, "32x32"), (69, 5016, 1720, True, "32x32"),
+    (700, 2052, 260, False, "32x64"), (700, 2052, 260, True, "32x64"),
+    (330, 1500, 260, False, "64x64"), (330, 1500, 260, True, "64x32"), (529, 1088, 260, False, "64x64"), (529, 1088, 260, True, "64x32"),
+    (529, 1088, 196, False, "64x32"), (1816, 524, 260, True, "64x32"), (1816, 524, 260, False, "64x32"),
+    (2050, 1028, 260, False, "64x64"),
+])
+def test_fp32_grids(m, n, k, kn, want):
+    assert ran(m, n, k, F32, kn=kn) == f"fp32_buffered {want}"
