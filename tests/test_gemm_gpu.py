@@ -284,8 +284,8 @@ def test_fp32_reference_known_answer(kernel, layout):
     assert orc.rel_frobenius(out.cpu().numpy(), ref) <= 1e-5
 
 
-# The last two take the 64 x 64 tiles (at least 512 of them), the others the
-# 64 x 32 tiles.
+# The last two take the 64 x 64 tiles (at least 512 of them) and 32 x 64, the
+# others 16 x 32.
 FP32_BUFFERED_SHAPES = [(1, 4, 4), (3, 8, 60), (64, 64, 64), (65, 68, 68), (130, 196, 132), (127, 192, 260),
                         (200, 256, 1028), (257, 132, 192), (1500, 1400, 68), (1090, 1028, 100)]
 
@@ -294,7 +294,7 @@ FP32_BUFFERED_SHAPES = [(1, 4, 4), (3, 8, 60), (64, 64, 64), (65, 68, 68), (130,
 def test_fp32_buffered_ragged(layout):
     """fp32_tiled on 16-byte rows (K % 4 == 0, N % 4 == 0 for B[K,N]): the
     buffered form, on edge tiles in M and N and K tails that are not a
-    multiple of the 32- or 64-wide K-tile, in both tile configurations;
+    multiple of the 32- or 64-wide K-tile, in three tile configurations;
     check_result against the float64 product and relative Frobenius <= 1e-5."""
     gen = torch.Generator().manual_seed(21)
     for m, n, k in FP32_BUFFERED_SHAPES:
@@ -311,7 +311,7 @@ def test_fp32_buffered_ragged(layout):
 
 
 @pytest.mark.parametrize("layout", [L.B_KN, L.B_NK], ids=["kn", "nk"])
-@pytest.mark.parametrize("m,n,k", [(130, 196, 132), (1500, 1400, 68)], ids=["tiles64x32", "tiles64x64"])
+@pytest.mark.parametrize("m,n,k", [(130, 196, 132), (1500, 1400, 68)], ids=["tiles16x32", "tiles64x64"])
 def test_fp32_buffered_padded_leading_dims(layout, m, n, k):
     """The buffered fp32 form through the C ABI with lda > K and ldb past the
     row length (K + 12 for W[N,K], N + 20 for B[K,N]): the padding holds NaN,
@@ -401,28 +401,34 @@ def test_workload_parity(name, m):
     _say(f"  {name} M={m}: {stats}")
 
 
-STAGED_GRIDS = [(600, 1000, 1000), (600, 1000, 2056), (1100, 2000, 1000), (2100, 2000, 1000), (2100, 4100, 1000),
-                (2100, 7000, 1000)]
+STAGED_GRIDS = [(600, 1000, 1000, "staged 64x64"), (600, 1000, 2056, "narrow 64x64"), (1100, 2000, 1000, "mid 128x128"),
+                (2100, 2000, 1000, "mid 128x256"), (2100, 4100, 1000, "wide 256x256"), (2100, 7000, 1000, "wide 256x256"),
+                (1579, 4992, 264, "staged 128x128"), (1100, 2000, 200, "staged 128x128"), (1000, 4333, 200, "staged 128x256")]
 
 
-@pytest.mark.parametrize("m,n,k", STAGED_GRIDS, ids=["40tiles-64x64", "40tiles-64x64-deep", "144tiles-spread",
-                                                     "wide136-128x256", "wide289-2deep", "wide476-128x256"])
+@pytest.mark.parametrize("m,n,k,form", STAGED_GRIDS, ids=["64x64-3deep", "64x64-long-k", "mid-128x128", "mid-128x256",
+                                                          "wide-153", "wide-252", "128x128-2deep", "128x128-3deep",
+                                                          "128x256"])
 @pytest.mark.parametrize("din,dout", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
                          ids=["bf16", "f16-f32"])
-def test_staged_ring_depths_ragged(m, n, k, din, dout):
-    """mfma_staged's tile choices: a grid of at most 128 tiles of 128 x 128
-    takes 64 x 64 tiles (3-deep ring, spread copies); up to 256 tiles 128 x
-    128 with the spread 3-deep ring; above that 128 x 256 tiles (8 waves,
-    3-deep ring, copies spread between the MFMAs) unless there are 257-384
-    of those, where 128 x 128 with a 2-deep ring takes over; each on ragged
-    M and N and a K that is not a multiple of the 64-wide K-tile (the last
-    tile is padded with zeros)."""
+def test_staged_ring_depths_ragged(m, n, k, form, din, dout):
+    """mfma_staged's tile choices: its own 64 x 64, 128 x 128 (3-deep ring, and
+    2-deep where 257-384 tiles of 128 x 256 are at most 512 of 128 x 128) and
+    128 x 256, the longer K-tiles of gemm_narrow.hip, the 128-row tiles of
+    gemm_mid.hip and the 256 x 256 ones of gemm_wide.hip; each on ragged M and
+    N and a K that is not a multiple of the 64-wide K-tile (the last tile is
+    padded with zeros), the first 100 rows bit for bit those of a launch of
+    their own."""
     _say(f"staged ring M={m} N={n} K={k} {NAME[din]}->{NAME[dout]}")
     gen = torch.Generator().manual_seed(m + n)
     a = torch.randn((m, k), generator=gen).to(din)
     w = (torch.randn((n, k), generator=gen) * 0.1).to(din)
-    out = G.gemm_with_kernel(a.to(DEV), w.to(DEV), L.KERNEL_MFMA_STAGED, dout, L.B_NK)
+    a_d, w_d = a.to(DEV), w.to(DEV)
+    out = G.gemm_with_kernel(a_d, w_d, L.KERNEL_MFMA_STAGED, dout, L.B_NK)
+    assert L.last_kernel() == f"mfma_{form}"
+    few = G.gemm_with_kernel(a_d[:100], w_d, L.KERNEL_MFMA_STAGED, dout, L.B_NK)
     torch.cuda.synchronize()
+    assert torch.equal(out[:100], few)
     rows = np.unique(np.concatenate([np.linspace(0, m - 1, 48).astype(int), np.arange(m - 16, m)]))
     _check_tolerance(out.cpu(), a, w, L.B_NK, dout, rows=rows)
 
@@ -432,18 +438,19 @@ def test_staged_tile_choices_same_bits(din):
     """Every tile choice of mfma_staged sums K in the same order, so a row's
     output does not depend on how many rows share the launch: with N = 4104
     and K = 1000, M = 100 / 600 / 1000 / 2100 select 64 x 64 tiles, 128 x 128
-    on the spread 3-deep ring, 128 x 256, and 128 x 128 on the 2-deep burst
-    ring, and the first 100 rows (fp32 outputs, so any reordering of the K
-    sum would show) are bit-identical across all four."""
+    and 128 x 256 of gemm_mid.hip, and 256 x 256, and the first 100 rows (fp32
+    outputs, so any reordering of the K sum would show) are bit-identical
+    across all four."""
     n, k, rows = 4104, 1000, 100
     gen = torch.Generator().manual_seed(4104)
     a = torch.randn((2100, k), generator=gen).to(din)
     w = (torch.randn((n, k), generator=gen) * 0.1).to(din)
     a_d, w_d = a.to(DEV), w.to(DEV)
     first = None
-    for m in (100, 600, 1000, 2100):
+    for m, form in ((100, "staged 64x64"), (600, "mid 128x128"), (1000, "mid 128x256"), (2100, "wide 256x256")):
         _say(f"staged tile choice M={m} N={n} K={k} {NAME[din]}->f32")
         out = G.gemm_with_kernel(a_d[:m], w_d, L.KERNEL_MFMA_STAGED, torch.float32, L.B_NK)
+        assert L.last_kernel() == f"mfma_{form}"
         torch.cuda.synchronize()
         head = out[:rows].cpu()
         if first is None:
@@ -458,8 +465,8 @@ def test_staged_tile_choices_same_bits(din):
 def test_staged_multi_round_same_bits(layout, dout):
     """A 128 x 256 grid of more than one round on the CUs (M = 512, N =
     33000: 4 x 129 = 516 tiles, a ragged last column of tiles): the first
-    100 rows equal, bit for bit, the same rows computed at M = 100 (64 x 64
-    tiles), every column, and sampled rows meet the tolerance."""
+    100 rows equal, bit for bit, the same rows computed at M = 100 (one round),
+    every column, and sampled rows meet the tolerance."""
     m, n, k, rows = 512, 33000, 256, 100
     gen = torch.Generator().manual_seed(33000)
     a = torch.randn((m, k), generator=gen).bfloat16()
@@ -1327,7 +1334,9 @@ def test_lm_head_random_inputs_match_torch_reference(m):
 # Sampled LM head (Sampler.forward without logits: greedy rows + Gumbel-max)
 # ---------------------------------------------------------------------------
 SAMPLE_CASES = ([(L.KERNEL_SPLITK_DECODE, m, n) for m in (1, 5, 32) for n in (1000, 70001)]
-                + [(L.KERNEL_MFMA_STAGED, m, 1000) for m in (1, 33, 300)])
+                + [(L.KERNEL_MFMA_STAGED, m, 1000) for m in (1, 33, 300)]
+                # 128 x 256 tiles: 157 of them, and 548 (more than 128 rows)
+                + [(L.KERNEL_MFMA_STAGED, 33, 40001), (L.KERNEL_MFMA_STAGED, 130, 70001)])
 
 
 def _sample_temps(m, gen):
@@ -1357,6 +1366,8 @@ def test_sample_admissible_against_oracle(kernel, m, n, din, rank):
     _say(f"sample {L.kernel_name(kernel)} {NAME[din]} M={m} N={n}")
     ldt = None if rank == "model" else torch.float32
     tokens, scores = G.gemm_sample_with_kernel(ad, wd, td, seed, offset, kernel, ldt)
+    if kernel == L.KERNEL_MFMA_STAGED:
+        assert L.last_kernel() == ("mfma_staged 128x256" if n > 1000 else "mfma_staged 128x128")
     g_tokens, g_values = G.gemm_argmax_with_kernel(ad, wd, kernel, ldt)
     torch.cuda.synchronize()
     tokens, scores = tokens.cpu().numpy(), scores.cpu().numpy()
@@ -1384,22 +1395,24 @@ def test_sample_admissible_against_oracle(kernel, m, n, din, rank):
         np.testing.assert_allclose(scores[~greedy], sc[~greedy], rtol=1e-5, atol=1e-3)
 
 
-@pytest.mark.parametrize("kernel,m", [(L.KERNEL_SPLITK_DECODE, 32), (L.KERNEL_MFMA_STAGED, 64)],
-                         ids=["splitk_decode", "mfma_staged"])
-def test_sample_noise_is_the_oracles_philox(kernel, m):
+@pytest.mark.parametrize("kernel,m,n", [(L.KERNEL_SPLITK_DECODE, 32, 64), (L.KERNEL_MFMA_STAGED, 64, 64),
+                                        (L.KERNEL_MFMA_STAGED, 40, 33001)],
+                         ids=["splitk_decode", "mfma_staged", "mfma_staged-128x256"])
+def test_sample_noise_is_the_oracles_philox(kernel, m, n):
     """At a huge temperature the score is -ln E (the logits vanish), so each
     row's token must carry the row's largest uniform u of the oracle's
     Philox stream: pins the device generator, its counter layout and word
-    choice bit for bit (64 columns: a wrong word or counter would miss the
-    maximum on most rows)."""
+    choice bit for bit (64 columns, or 129 tiles of 256 with a last one of
+    233: a wrong word or counter would miss the maximum on most rows)."""
     gen = torch.Generator().manual_seed(5)
-    n, k = 64, 64
+    k = 64
     a = torch.randn((m, k), generator=gen).bfloat16()
     w = (torch.randn((n, k), generator=gen) * 0.1).bfloat16()
     temps = torch.full((m,), 1e30)
     seed, offset = 0xDEADBEEF12345678, 99
     _say(f"sample noise {L.kernel_name(kernel)} M={m}")
     tokens, _ = G.gemm_sample_with_kernel(a.to(DEV), w.to(DEV), temps.to(DEV), seed, offset, kernel)
+    assert n == 64 or L.last_kernel() == "mfma_staged 128x256"
     torch.cuda.synchronize()
     u = orc.sample_uniform(m, n, seed, offset)
     tokens = tokens.cpu().numpy()

@@ -39,6 +39,7 @@ def test_mid_tiles(m, n, k, din, dout):
     ad, wd = a.to(DEV), w.to(DEV)
     _say(f"mid M={m} N={n} K={k} {NAME[din]}->{NAME[dout]}")
     out = G.gemm_with_kernel(ad, wd, L.KERNEL_MFMA_STAGED, dout)
+    assert L.last_kernel() == f"mfma_mid 128x{128 if n in (1001, 2001, 1920) else 256}"
     for r0 in (0, 100, m - 200, m - 100):
         part = G.gemm_with_kernel(ad[r0:r0 + 100], wd, L.KERNEL_MFMA_STAGED, dout)
         torch.cuda.synchronize()
@@ -62,6 +63,7 @@ def test_mid_tiles_silu(norm, dout):
     else:
         run = lambda x: G.gemm_silu_mul_with_kernel(x, wd, L.KERNEL_MFMA_STAGED, dout)  # noqa: E731
     out = run(ad)
+    assert L.last_kernel() == "mfma_mid 128x128"
     for r0 in (0, 100, m - 100):
         part = run(ad[r0:r0 + 100])
         torch.cuda.synchronize()

@@ -265,19 +265,22 @@ def test_add_rmsnorm_prologue_kernel_path(m, silu):
         _check_add_norm(out, res_out, h, r, nw, w, 1e-5, torch.bfloat16, torch.bfloat16)
 
 
-@pytest.mark.parametrize("m,n,silu", [(1500, 2000, False), (2100, 2000, False), (2100, 1000, True),
-                                      (2100, 4100, False)],
-                         ids=["128x128-spread", "128x256", "128x256-silu", "128x128-2deep"])
-def test_add_rmsnorm_row_scale_large_grids(m, n, silu):
-    """The row-scaled epilogue on mfma_staged's large-grid tiles: 192 tiles
-    of 128 x 128 (3-deep ring, spread copies), 136 tiles of 128 x 256 (8
-    waves, spread copies; plain and with SiLU-and-mul) and 289 (where 128 x
-    128 with a 2-deep ring takes over); ragged M, N and K."""
+@pytest.mark.parametrize("m,n,k,silu,form", [
+    (1500, 2000, 1000, False, "mid 128x128"), (2100, 2000, 1000, False, "mid 128x256"),
+    (2100, 1000, 1000, True, "mid 128x128"), (2100, 4100, 1000, False, "wide 256x256"),
+    (2100, 2050, 264, True, "wide 256x128"), (1100, 2000, 200, False, "staged 128x128"),
+    (1579, 4992, 264, False, "staged 128x128"), (500, 1029, 1800, False, "narrow 64x64"),
+    (200, 3333, 320, True, "narrow 64x32"), (200, 3333, 264, True, "staged 64x64")],
+    ids=["mid-128x128", "mid-128x256", "mid-silu", "wide", "wide-silu", "128x128-3deep", "128x128-2deep", "narrow-64x64",
+         "narrow-silu", "64x128-silu"])
+def test_add_rmsnorm_row_scale_large_grids(m, n, k, silu, form):
+    """The row-scaled epilogue of every tile of mfma_staged beyond its smallest,
+    plain and with SiLU-and-mul; ragged M, N and K."""
     gen = torch.Generator().manual_seed(m + n)
-    k = 1000
     h, r, nw, w = _norm_inputs(m, 2 * n if silu else n, k, torch.bfloat16, gen)
     _say(f"add_rmsnorm large grid M={m} N={n} silu={silu}")
     out, res_out = K.gemm_add_rmsnorm(h.to(DEV), r.to(DEV), nw.to(DEV), w.to(DEV), 1e-5, silu_mul=silu)
+    assert L.last_kernel() == f"mfma_{form}"
     torch.cuda.synchronize()
     if silu:
         _check_add_norm_silu(out, res_out, h, r, nw, w, 1e-5, torch.bfloat16, torch.bfloat16)

@@ -52,6 +52,7 @@ def test_ragged_tiles(m, n, k, layout, din, dout):
         c = torch.full((m, ldc), 7.0, dtype=dout, device=DEV)
         L.gemm_raw(ap, bp, c.data_ptr(), m, n, k, lda, ldb, ldc, layout, CODE[din], CODE[dout],
                    torch.cuda.current_stream().cuda_stream, kernel=L.KERNEL_MFMA_DIRECT)
+        assert L.last_kernel().startswith("mfma_direct" if k <= 16 else "mfma_ragged")
         torch.cuda.synchronize()
         _check_tolerance(c[:, :n].cpu(), a, b, layout, dout)
         assert bool((c[:, n:] == 7.0).all()), "a padding column was written"

@@ -19,9 +19,11 @@ G = importlib.import_module("inference_systems_amd.kernels.gemm")
 BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 
 
-# 32 x 32 tiles, 64 x 64 (mfma_staged), 128 x 128 and 128 x 256 (gemm_mid.hip),
-# 256 x 256.
-@pytest.mark.parametrize("m,k", [(70, 136), (1100, 136), (1100, 264), (2300, 264), (5000, 264)], ids=lambda v: str(v))
+FORMS = {(70, 136): "narrow 32x32", (1100, 136): "staged 64x64", (1100, 264): "staged 64x64",
+         (2200, 264): "mid 128x128", (2300, 264): "mid 128x256", (5000, 264): "wide 256x256"}
+
+
+@pytest.mark.parametrize("m,k", FORMS, ids=lambda v: str(v))
 @pytest.mark.parametrize("n", [1032, 1031], ids=["even", "odd"])
 @pytest.mark.parametrize("din,dout", [(BF16, BF16), (F16, F32)], ids=["bf16", "f16-f32"])
 def test_unaligned_rows(m, n, k, din, dout):
@@ -37,6 +39,7 @@ def test_unaligned_rows(m, n, k, din, dout):
                    torch.cuda.current_stream().cuda_stream, kernel=L.KERNEL_MFMA_STAGED)
 
     run(full, full.shape[1])
+    assert L.last_kernel() == f"mfma_{FORMS[m, k]}"
     for ldc, first in ((n + 1, 0), (n + 2, 0), (n + 4, 1), (n + 4, 2)):
         buf = torch.full((first + m * ldc,), 7.0, dtype=dout, device=DEV)
         c = buf[first:].view(m, ldc)

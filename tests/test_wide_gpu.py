@@ -1,6 +1,6 @@
 """GPU tests of mfma_staged's 256 x 256 tiles (csrc/gemm_wide.hip): grids that
 take them at the edges of tiles, K-tiles and the C tile's store, against the
-same rows computed 100 at a time (64 x 64 tiles, which sum K in the same
+same rows computed 100 at a time (smaller tiles, which sum K in the same
 order, so every bit is equal) and against the oracle."""
 from __future__ import annotations
 
@@ -31,18 +31,21 @@ def _inputs(m, rows, k, dtype):
     return torch.randn((m, k), generator=gen).to(dtype), (torch.randn((rows, k), generator=gen) * 0.1).to(dtype)
 
 
-# 168-252 tiles of 256 x 256.  N = 3333 and 12290 store element by element in
-# the last column of tiles (and, with 2-byte outputs, in every tile: rows are
-# not 16-byte aligned); K = 256 / 264 / 320 / 328 is 4-6 K-tiles with tails of
-# 0, 8, 0 and 8.
+# 160-192 tiles of 256 x 256, and 400 (a round and a part).  N = 3333 and 3334
+# store element by element in the last column of tiles (and, with 2-byte outputs,
+# in every tile: rows are not 16-byte aligned); K = 256 / 264 / 320 / 328 is 4-6
+# K-tiles with tails of 0, 8, 0 and 8.  1301 x 12290 (294 tiles) runs 128-row tiles:
+# 256 x 256 would leave most of a second round idle.
 @pytest.mark.parametrize("m,n,k,din,dout", [
     (2900, 3333, 264, BF16, BF16), (2900, 3333, 264, BF16, F32), (4096, 2560, 256, BF16, BF16),
-    (1301, 12290, 328, F16, F16), (2817, 4096, 320, F16, F32)], ids=lambda v: NAME.get(v, v))
+    (1301, 12290, 328, F16, F16), (2817, 4096, 320, F16, F32), (2900, 3334, 328, F16, F16),
+    (5000, 5000, 328, BF16, BF16)], ids=lambda v: NAME.get(v, v))
 def test_wide_tiles(m, n, k, din, dout):
     a, w = _inputs(m, n, k, din)
     ad, wd = a.to(DEV), w.to(DEV)
     _say(f"wide M={m} N={n} K={k} {NAME[din]}->{NAME[dout]}")
     out = G.gemm_with_kernel(ad, wd, L.KERNEL_MFMA_STAGED, dout)
+    assert L.last_kernel() == ("mfma_mid 128x256" if n == 12290 else "mfma_wide 256x256")
     for r0, r1 in _blocks(m):
         part = G.gemm_with_kernel(ad[r0:r1], wd, L.KERNEL_MFMA_STAGED, dout)
         torch.cuda.synchronize()
@@ -69,6 +72,7 @@ def test_wide_tiles_silu(norm, dout):
         return G.gemm_silu_mul_with_kernel(ad[r0:r1], wd, L.KERNEL_MFMA_STAGED, dout)
 
     out = run(0, m)
+    assert L.last_kernel() == "mfma_wide 256x128"
     for r0, r1 in _blocks(m):
         part = run(r0, r1)
         torch.cuda.synchronize()
