@@ -72,10 +72,11 @@ constexpr int64_t kDecodeMaxM = 32;
 
 // The plain GEMM also runs on splitk_decode up to M = 64 when W has fewer
 // than 65536 rows.  The table picks it there for narrow problems, where
-// mfma_staged leaves CUs idle (bf16, M = 64, against its smallest tiles: N =
-// 1024, K = 3584 6.7 against 8.4 us; N = 2048, K = 2048 6.1 against 6.3 us; they
-// are level at N = 4096), and not from 16384 rows or, above 4096 rows, beyond
-// K = 1024 (N = 12288, K = 2048: 14.3 against 11.6 us).
+// mfma_staged leaves CUs idle (bf16, M = 64, W from HBM, against its smallest
+// tiles, us: N = 1024, K = 1024 / 3584 3.4 / 5.6 against 5.0 / 10.5; N = 2048, K =
+// 2048 5.5 against 7.3; about level at N = 4096, K = 1024 / 4096 5.0 / 12.7 against
+// 5.2 / 12.2, and N = 8224, K = 1024 8.3 against 7.9), and not from 16384 rows or,
+// above 4096 rows, beyond K = 1024 (N = 12288, K = 2048: 14.3 against 11.6 us).
 constexpr int64_t kSplitkPlainMaxM = 64;
 constexpr int64_t kSplitkPlainMaxRows = 65535;
 constexpr int64_t kSplitkPlainNarrowN = 4096;
@@ -126,11 +127,13 @@ int select(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int b_layo
         return NANOVLLM_GEMM_KERNEL_MFMA_STAGED;
     }
     // B[K,N] (the reference bench's layout): splitk_decode up to M = 32 and
-    // up to M = 64 on at most 4096 columns, the staged kernel above.  On the
-    // reference's shape matrix (bf16, fp32 out) splitk_decode took M = 1 / 16
-    // from 6.2-9.9 us (staged) to 3.7-4.6 us, and 64 x 1024 x 2048 / 3584
-    // from 10.0 / 15.8 to 8.1 / 10.8 us; at 64 x 6144 / 7168 (96 / 112
-    // workgroups of 64 columns) it ran 6.8 / 7.0 against 6.6 / 6.7 us.
+    // up to M = 64 on at most 4096 columns, the staged kernel above (bf16, fp32
+    // out, B from HBM, against mfma_staged's 32 x 64 tiles, us: M = 1 / 16 / 32, 1024
+    // x 2048 6.7 / 7.2 / 8.2 against 10.7 / 11.6 / 12.3, 6144 x 1024 5.3 / 5.7 / 6.7
+    // against 7.4 / 8.0 / 8.4; M = 64, 1024 x 2048 / 3584 11.8 / 17.0 against 12.1 /
+    // 18.8, 6144 x 1024 9.2 against 8.4).  Between, M = 64 on 2048 to 4096 columns,
+    // the tiles are a little ahead (2048 x 2048 12.0 against 11.8, 4096 x 1024 8.7 /
+    // 8.0, 4096 x 4096 25.8 / 21.5).
     if (kn_vector_ok(n, k, lda, ldb, b_layout, aligned16)) {
         if (m <= kDecodeMaxM || (m <= kSplitkPlainMaxM && n <= kSplitkPlainNarrowN))
             return NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
@@ -221,10 +224,11 @@ int select_silu_mul(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldw, i
     // 1024) splitk_decode's whole-line copies take 4.9 us against 5.2 us for
     // gemv_decode streaming the gate and up rows.
     if (m <= kDecodeMaxM) return NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
-    // 33 <= M <= 64: mfma_staged's SiLU grid is one row of 64 x 128 tiles;
-    // splitk_decode spreads the gate/up pairs over 2n / 32 workgroups (bf16,
-    // K = 1024, M = 64: n = 3584 4.7 against 9.2 us, n = 8192 9.7 against
-    // 11.9 us; K = 2048, n = 3584: 8.1 against 15.1 us).
+    // 33 <= M <= 64: splitk_decode spreads the gate/up pairs over 2n / 32
+    // workgroups (bf16, W from HBM, M = 64, against mfma_staged's tiles of 32 x 32
+    // and 64 x 32 outputs, us: K = 1024 / 2048, n = 2048 5.6 / 8.8 against 6.8 / 10.1,
+    // n = 3584 6.4 / 10.7 against 7.1 / 10.9).  Near the upper end the tiles are
+    // ahead (n = 8192 12.2 / 19.6 against 8.9 / 17.0).
     if (m <= kSplitkPlainMaxM && 2 * n <= kSplitkSiluMaxRows) return NANOVLLM_GEMM_KERNEL_SPLITK_DECODE;
     return NANOVLLM_GEMM_KERNEL_MFMA_STAGED;
 }

@@ -20,10 +20,12 @@
 //   * line L is accumulated into K partition L % PARTS, each wave owning
 //     PARTS / WAVES partitions, and the partition sums are added in LDS in
 //     partition order (deterministic, no atomics, no workspace) and written
-//     once.  The order of every sum depends on PARTS alone, so all
+//     once.  The order of every sum over K depends on PARTS alone, so all
 //     configurations with PARTS = 16 (every W of fewer than 65536 rows)
 //     give bit-identical results for a given row of A and row of W, whatever
-//     N: a merged projection equals its separate parts.
+//     N: a merged projection equals its separate parts.  The norm's sum of
+//     squares is added up per wave, so the row scale goes by WAVES too (8 or 16
+//     by the configuration).
 // It replaces the reference's cuBLAS fallback for decode shapes and the
 // M == 16 direct-WMMA special case (cuda_kernels/gemm/src/gemm_bench.cu:260-273).
 #include "decode_kernels.hpp"
@@ -46,10 +48,9 @@ namespace {
 //     workgroups, with 16 waves along K (M = 1 / 16: 4.7 / 6.6 us, against
 //     7.0 / 9.0 us with 32 rows).  Where that leaves CUs idle, the rows of A
 //     are spread over workgroups too (launch_rows);
-//   * rows >= 65536 (the LM head, N = 151936, K = 1024): M = 1 runs the
-//     register-loading kernel (48.4 us; with a prologue, the M <= 8
-//     configuration); M = 8 / 16 / 32: 53.5 / 57.5 / 63.9 us (61.2 / 65.7 /
-//     75.8 us with register loading).
+//   * rows >= 65536 (the LM head, N = 151936, K = 1024): M = 1 on the
+//     configuration of M = 2-8; M = 8 / 16 / 32: 53.5 / 57.5 / 63.9 us (61.2 /
+//     65.7 / 75.8 us with register loading).
 //   * 33 <= M <= 64 (the plain GEMM only, below 65536 rows): A's copies now
 //     outweigh W's, so 8 waves and 8 K partitions above 2048 rows, 16 / 32 /
 //     48 rows per workgroup up to 4096 / 8192 / 65535 rows; from 16384 rows
@@ -229,7 +230,7 @@ int launch_rows(const Problem& p, hipStream_t s) {
     // each (every line of a 1024-wide K in flight at once); on wider W the
     // configuration whose busiest CU streams the fewest W rows, then the one
     // that needs the fewest rounds of resident workgroups, then the fewest
-    // workgroups (see pick_rows).  A grid one workgroup past a round pays
+    // workgroups (RowsChoice).  A grid one workgroup past a round pays
     // for a second one.  Measured on MI355X (W streamed from HBM, bench.py
     // --decode-sweep), M = 4 / 8 / 16 / 32: N = 8224 (257 workgroups of 32
     // rows) 5.74 / 5.91 / 7.31 / 8.45 us with 32 rows throughout, 5.31 /

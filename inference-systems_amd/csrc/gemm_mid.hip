@@ -68,9 +68,9 @@ __global__ __launch_bounds__(kThreads) void mfma_mid_kernel(
     const int64_t m0 = int64_t(tm) * kBM, n0 = int64_t(tn) * BNO;
 
     // Copy instruction j of a wave fills 8 LDS rows, lane L row L / 8, position
-    // L % 8, which holds logical chunk (L % 8) ^ ((row >> 1) & 7).  j < 8: W
-    // rows (EPI_SILU_MUL alternates 32 gate rows and the 32 up rows of the same
-    // output columns); j >= 8: A rows.
+    // L % 8, which holds logical chunk (L % 8) ^ ((row >> 1) & 7).  j <
+    // kWCopies: W rows (EPI_SILU_MUL alternates 32 gate rows and the 32 up rows
+    // of the same output columns); the others: A rows.
     auto copy_row = [&](int j) { return j < kWCopies ? kBM + 8 * (kWCopies * wave + j) : 8 * ((kCopies - kWCopies) * wave + j - kWCopies); };
     const uint16_t* abase = a + m0 * lda;
     const uint16_t* wbase = w + n0 * ldb;
