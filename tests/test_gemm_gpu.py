@@ -484,8 +484,8 @@ def test_staged_multi_round_same_bits(layout, dout):
 
 @pytest.mark.parametrize("din", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_staged_square256_same_bits(din):
-    """fp32 logits over a W larger than the Infinity Cache take 256 x 256
-    tiles whose C tile leaves LDS in two passes of 128 rows: M = 500, N =
+    """fp32 logits on the 256 x 256 tiles of gemm_wide.hip, whose C tile leaves
+    LDS in two passes of 128 rows: M = 500, N =
     140001, K = 1000 (W 280 MB; 2 x 547 tiles, a ragged last column, a
     last tile row that ends inside its second pass, a K tail).  Rows 0-99
     and 400-499 equal, bit for bit, the same rows computed alone (M = 100:
@@ -498,6 +498,7 @@ def test_staged_square256_same_bits(din):
     a_d, w_d = a.to(DEV), w.to(DEV)
     _say(f"staged 256x256 M={m} N={n} K={k} {NAME[din]}->f32")
     full = G.gemm_with_kernel(a_d, w_d, L.KERNEL_MFMA_STAGED, torch.float32, L.B_NK)
+    assert L.last_kernel() == "mfma_wide 256x256"
     torch.cuda.synchronize()
     for r0 in (0, 400):
         part = G.gemm_with_kernel(a_d[r0:r0 + 100], w_d, L.KERNEL_MFMA_STAGED, torch.float32, L.B_NK)
